@@ -369,12 +369,12 @@ int lbm_links_apply_sets(void* d_f, const lbm_layout* layout, const lbm_link_set
                          void* stream);
 
 /*
- * nsteps time steps of a 2D scheme on the wrap path (a periodic box, or every link
- * list folded into bbmask / bbtab with bbtab_rel set), steps_per_launch (<= 16) of
- * them per launch: each workgroup loads a tile_m x tile_i tile of the interior with
- * a halo of steps_per_launch cells into LDS and advances it there, with the
- * per-cell arithmetic of lbm_gen_step (the same bits); the remaining
- * nsteps % steps_per_launch steps run as lbm_gen_step launches.  This is
+ * nsteps time steps of a 1D or 2D scheme on the wrap path (a periodic box, or every
+ * link list folded into bbmask / bbtab with bbtab_rel set), at most steps_per_launch
+ * (<= 16 in 2D, <= 64 in 1D) of them per launch: each workgroup loads a
+ * tile_m x tile_i tile of the interior (tile_m = 1 in 1D) with a halo of
+ * steps_per_launch cells into LDS and advances it there, with the per-cell arithmetic
+ * of lbm_gen_step (the same bits).  This is
  * pylbm/simulation.py:392-420 repeated, for grids whose step is too small to fill
  * the GPU.  *parity as for lbm_gen_run; params->t advances by nsteps dt.
  */

@@ -426,7 +426,8 @@ using namespace lbm;
 #ifndef TB_THREADS
 #define TB_THREADS 1024                // threads of a temporally blocked workgroup
 #endif
-#define TB_MAX_NT 16                   // steps per temporally blocked launch, at most
+#define TB_MAX_NT (DIM == 1 ? 64 : 16) // steps per temporally blocked launch, at most
+#define TB_PLANE_1D 256                // cells of a 1D region, at most
 #define TB_MASK %(bbsub_ok)d                    // folded links possible: mask words kept in LDS
 
 namespace {
@@ -939,7 +940,7 @@ int lbm_gen_run_blocked(void* d_f, void* d_fnew, const lbm_layout* layout, lbm_p
                         int64_t nsteps, int steps_per_launch, int tile_m, int tile_i, int* parity,
                         void* stream) {
   LBM_REQUIRE(params && layout && parity, "NULL argument");
-  LBM_REQUIRE(DIM == 2, "temporal blocking is generated for 2D schemes only (this one is %%dD)", DIM);
+  LBM_REQUIRE(DIM <= 2, "temporal blocking is generated for 1D and 2D schemes only (this one is %%dD)", DIM);
   LBM_REQUIRE(TB_UNIT_VELOCITIES, "temporal blocking needs velocity components in {-1, 0, 1}");
   LBM_REQUIRE(steps_per_launch >= 1 && steps_per_launch <= TB_MAX_NT, "steps per launch out of [1, %%d]",
               TB_MAX_NT);
@@ -951,26 +952,24 @@ int lbm_gen_run_blocked(void* d_f, void* d_fnew, const lbm_layout* layout, lbm_p
   hipStream_t s = (hipStream_t)stream;
   void* a = d_f;
   void* b = d_fnew;
-  int64_t done = 0;
-  const int64_t blocks = nsteps / steps_per_launch;
-  for (int64_t it = 0; it < blocks; ++it) {
+  // nsteps in launches of at most steps_per_launch steps, as even as they come: 200
+  // steps at most 6 at a time are 32 launches of 6 and 2 of 4, not 33 and two steps
+  const int64_t launches = (nsteps + steps_per_launch - 1) / steps_per_launch;
+  for (int64_t it = 0; it < launches; ++it) {
+    const int nt = (int)(nsteps * (it + 1) / launches - nsteps * it / launches);
     int rc = 0;
-    LBM_DISPATCH_BLOCKED(layout->storage, tb_launch, a, b, layout, params, steps_per_launch, tile_m, tile_i, s, rc);
+    if (nt > 1) {
+      LBM_DISPATCH_BLOCKED(layout->storage, tb_launch, a, b, layout, params, nt, tile_m, tile_i, s, rc);
+    } else {
+      rc = lbm_gen_step(a, b, layout, params, 1, stream);
+      params->t += params->dt;
+    }
     if (rc) return rc;
     void* tmp = a;
     a = b;
     b = tmp;
-    done += steps_per_launch;
   }
-  for (; done < nsteps; ++done) {
-    int rc = lbm_gen_step(a, b, layout, params, 1, stream);
-    if (rc) return rc;
-    void* tmp = a;
-    a = b;
-    b = tmp;
-    params->t += params->dt;
-  }
-  *parity = (int)(blocks & 1) ^ (int)((nsteps - blocks * steps_per_launch) & 1);
+  *parity = (int)(launches & 1);
   return 0;
 }
 
@@ -1034,6 +1033,7 @@ __device__ __forceinline__ int wrap_near(int x, int n) {
 // the 16-bit immediate offset.
 template <typename S>
 __host__ __device__ constexpr int tb_plane() {
+  if (DIM == 1) return TB_PLANE_1D;
   constexpr int a = (160 * 1024) / (2 * NS * (int)sizeof(S) + 12);
   constexpr int b = NS > 1 ? 65528 / ((NS - 1) * (int)sizeof(S)) : a;
   return a < b ? a : b;
@@ -1046,7 +1046,8 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   using C = typename Codec<S>::C;
   constexpr bool DEV = Codec<S>::kind != LBM_F64;
   extern __shared__ uint4 tb_smem[];
-  const int RW = t.tm + 2 * t.nt, RI = t.ti + 2 * t.nt, RN = RW * RI;
+  constexpr int MH = DIM == 2;   // the mid axis has a halo (a 1D region is one row)
+  const int RW = t.tm + 2 * t.nt * MH, RI = t.ti + 2 * t.nt, RN = RW * RI;
   constexpr int RC = tb_plane<S>();   // plane stride (cells), RN <= RC
   S* cur = reinterpret_cast<S*>(tb_smem);
   S* nxt = cur + NS * RC;
@@ -1058,7 +1059,7 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   uint32_t* tbase_l = tbits + RN;
   const bool table = TB_MASK && a.bbmask && a.bbtab_bits;
   (void)msk; (void)tbits; (void)tbase_l; (void)table;
-  const int m0 = (int)(blockIdx.x / t.tiles_i) * t.tm - t.nt;
+  const int m0 = (int)(blockIdx.x / t.tiles_i) * t.tm - t.nt * MH;
   const int i0 = (int)(blockIdx.x %% t.tiles_i) * t.ti - t.nt;
   const C half_dt = a.half_dt;
   (void)half_dt;
@@ -1085,16 +1086,16 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   for (int s = 1; s <= t.nt; ++s) {
     const C tt = t.times[s - 1];
     (void)tt;
-    const int WC = RI - 2 * s, HC = RW - 2 * s;
+    const int WC = RI - 2 * s, HC = RW - 2 * s * MH;
     // the cells of the shrunk region in row-major order, blockDim.x apart: the
     // (row, column) of the next one follow by adding (dq, dr) with a carry, and its
     // region index by adding dl, plus dc on a carry (no multiply per cell)
     const int dq = (int)blockDim.x / WC, dr = (int)blockDim.x - dq * WC;
     int rr = (int)threadIdx.x / WC, qq = (int)threadIdx.x - rr * WC;
     const int dl = dq * RI + dr, dc = RI - WC;
-    int lnext = (s + rr) * RI + s + qq;
+    int lnext = (s * MH + rr) * RI + s + qq;
     for (int c = threadIdx.x; c < WC * HC; c += blockDim.x) {
-      const int lr = s + rr, lc = s + qq;
+      const int lr = s * MH + rr, lc = s + qq;
       const int lcell = lnext;
       qq += dr;
       rr += dq;
@@ -1133,7 +1134,7 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
     nxt = tmp;
   }
   for (int c = threadIdx.x; c < t.tm * t.ti; c += blockDim.x) {
-    const int lr = t.nt + c / t.ti, lc = t.nt + c %% t.ti;
+    const int lr = t.nt * MH + c / t.ti, lc = t.nt + c %% t.ti;
     const int gm = m0 + lr, gi = i0 + lc;
     if (gm >= a.nin[1] || gi >= a.nin[2]) continue;
     const int64_t dst = (int64_t)(a.halo[0] * a.n1 + gm + a.halo[1]) * a.rs + a.lead + gi + a.halo[2];
@@ -1152,7 +1153,7 @@ static int tb_launch(void* f, void* fn, const lbm_layout* L, lbm_params* p, int 
   StepArgs<C> a;
   int rc = make_args<C>(L, p, &a);
   if (rc) return rc;
-  LBM_REQUIRE(a.nin[1] >= tm && a.nin[2] >= ti && a.nin[1] >= nt && a.nin[2] >= nt,
+  LBM_REQUIRE(a.nin[1] >= tm && a.nin[2] >= ti && (DIM == 1 || a.nin[1] >= nt) && a.nin[2] >= nt,
               "tile %%d x %%d / %%d steps larger than the interior", tm, ti, nt);
   TbArgs<C> t{};
   t.nt = nt;
@@ -1164,7 +1165,9 @@ static int tb_launch(void* f, void* fn, const lbm_layout* L, lbm_params* p, int 
     p->t += p->dt;
   }
   const int tiles_m = (a.nin[1] + tm - 1) / tm;
-  const size_t region = (size_t)(tm + 2 * nt) * (ti + 2 * nt);
+  const size_t region = (size_t)(DIM == 1 ? tm : tm + 2 * nt) * (ti + 2 * nt);
+  // a thread per region cell, at most TB_THREADS: a 1D region needs few waves
+  const unsigned threads = DIM == 1 ? (unsigned)((region + 63) / 64 * 64) : TB_THREADS;
   const bool mask = TB_MASK && p->bbmask, table = mask && p->bbtab_bits;
   LBM_REQUIRE(region <= (size_t)tb_plane<S>(), "tile region of %%zu cells exceeds the %%d cells of a plane",
               region, tb_plane<S>());
@@ -1172,7 +1175,7 @@ static int tb_launch(void* f, void* fn, const lbm_layout* L, lbm_params* p, int 
   LBM_REQUIRE(lds <= 160 * 1024, "tile needs %%zu bytes of LDS", lds);
   LBM_CHECK_HIP(hipFuncSetAttribute((const void*)tb_step<S>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds));
-  tb_step<S><<<dim3((unsigned)(tiles_m * t.tiles_i)), dim3(TB_THREADS), lds, s>>>((const S*)f, (S*)fn, a, t);
+  tb_step<S><<<dim3((unsigned)(tiles_m * t.tiles_i)), dim3(threads), lds, s>>>((const S*)f, (S*)fn, a, t);
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1367,7 +1370,7 @@ def generate_source(spec: KernelSpec) -> str:
     vel_txt = ", ".join("{%d, %d, %d}" % v for v in vel)
 
     # ------------------------------------------- temporally blocked kernel (2D)
-    if dim == 2:
+    if dim <= 2:
         tb_loads = ["S %s;" % ", ".join("L%d[1]" % k for k in range(ns))]
         tb_loads += ["L%d[0] = cur[%d * RC + lcell - (%d * RI + %d)];" % (k, k, vel[k][1], vel[k][2])
                      for k in range(ns)]

@@ -44,6 +44,13 @@ LBM_F64 = rtm.LBM_F64
 # waves, and 126,620 of them spread over C4's waves cost 37 us per step against a
 # 4.5 us launch of the same copies (MI355X); smaller tables save their launches.
 FOLD_TABLE_MAX = 1 << 16
+# Temporally blocked run in 1D: (steps per launch, cells per tile); a tile and its halo
+# of steps cells on both sides fill one region of TB_PLANE_1D cells (the generated
+# module's constant of the same name).  A 1D step is launch and latency: the 5000-cell
+# FP64 shock tube (3 x D1Q2, Neumann ends) takes 4.1 us per step with one launch each
+# and 1.4 us this way.
+TB_SHAPE_1D = (64, 128)
+TB_PLANE_1D = 256
 
 
 def _canon_velocities(spec, box_label=None):
@@ -533,10 +540,10 @@ class Simulation:
 
     def _relative_sources(self, cell, src):
         """Table sources relative to their pulling cell, for the temporally blocked run
-        (2D): population | (mid offset + 128) << 8 | (inner offset + 128) << 16, the
+        (1D and 2D): population | (mid offset + 128) << 8 | (inner offset + 128) << 16, the
         offsets taken through the periodic wrap; None when a source is farther than
-        one cell away or the scheme is not 2D."""
-        if self.dim != 2 or src.size == 0:
+        one cell away or the scheme is 3D."""
+        if self.dim > 2 or src.size == 0:
             return None
         L, n, h, nin = self._fold_layout()
         k, o, m, i = _unflat_fn(np.asarray(src, dtype=np.int64), L)
@@ -734,7 +741,7 @@ class Simulation:
         self.params.t = self.t
         parity = ctypes.c_int(0)
         tb = self._blocking_shape() if fold else None
-        if tb is not None and nsteps >= tb[0]:
+        if tb is not None and nsteps > 1:
             nt, tm, ti = tb
             self._check(self.module.lbm_gen_run_blocked(ctypes.c_void_p(c.F.ptr), ctypes.c_void_p(c.Fnew.ptr),
                                                         ctypes.byref(c.F.layout), ctypes.byref(self.params),
@@ -759,9 +766,9 @@ class Simulation:
 
     def _blocking_shape(self):
         """(steps per launch, tile rows, tile columns) of the temporally blocked run, or
-        None: 2D schemes on the wrap path (periodic, or every list folded with its
-        table sources within one cell) whose grid is small enough that a step does not
-        fill the GPU (at most 2^21 cells).  The tile and its halo live in LDS: two
+        None: 1D and 2D schemes on the wrap path (periodic, or every list folded with
+        its table sources within one cell), in 2D on grids small enough that a step
+        does not fill the GPU (at most 2^21 cells).  The tile and its halo live in LDS: two
         copies of ns populations per cell in planes of a fixed size (the most cells
         that fit the 160 KiB of a CU with the mask and table words), and the region
         has to fit one plane.  The preferred shapes were measured on MI355X
@@ -769,7 +776,7 @@ class Simulation:
         formats, 4 steps of 16 x 32 tiles for FP64, 6 steps of 8 x 16 tiles for FP64
         grids of at most 2^15 cells (more tiles than CUs matter more there than the
         recomputed halo); larger schemes shrink the tile until it fits."""
-        if not self.temporal_blocking or self.dim != 2 or not self._wrap:
+        if not self.temporal_blocking or self.dim > 2 or not self._wrap:
             return None
         if np.any(np.abs(np.asarray(self.scheme.stencil.get_all_velocities())) > 1):
             return None
@@ -777,6 +784,12 @@ class Simulation:
                                                                       not self.params.bbtab_rel2):
             return None
         nin = [int(x) for x in self.domain.shape_in]
+        if self.dim == 1:
+            nt, ti = TB_SHAPE_1D
+            if 2 * self.ns * TB_PLANE_1D * self.container.F.layout.elem_size + 12 * TB_PLANE_1D > 160 * 1024:
+                return None
+            nt = min(nt, nin[0])
+            return (nt, 1, min(ti, nin[0])) if nt >= 2 else None
         cells = nin[0] * nin[1]
         if cells > (1 << 21):
             return None
