@@ -428,7 +428,8 @@ using namespace lbm;
 #endif
 #define TB_MAX_NT (DIM == 1 ? 64 : 16) // steps per temporally blocked launch, at most
 #define TB_PLANE_1D 256                // cells of a 1D region, at most
-#define TB_MASK %(bbsub_ok)d                    // folded links possible: mask words kept in LDS
+#define TB_MASK %(bbsub_ok)d                    // folded links possible
+#define TB_LINKS 4                     // folded links a thread of a blocked workgroup holds
 
 namespace {
 
@@ -1009,8 +1010,23 @@ _TB_KERNEL = r"""// ------------------------------------------------ temporally 
 // periodic box, or every link list folded into the mask / table), then for
 // s = 1 .. nt computes the cells of the region shrunk by s from the values of
 // step s - 1 with the per-cell arithmetic of fused_step (the same generated
-// lines, so the same bits), and finally stores the tile.  Folded links read their
-// sources at the offsets bbtab_rel gives relative to the pulling cell.
+// lines, so the same bits), and finally stores the tile.
+//
+// Folded links.  The link of population k at cell x gives the value that x pulls
+// from (k, x - v_k), and no other cell pulls that slot, so a workgroup applies its
+// links as pylbm's lists do: before each step every link's value is written into its
+// slot of the LDS region, and the cells then pull without looking at a mask.  The
+// load phase collects the region's links in a list (an LDS counter), one thread takes
+// TB_LINKS of them at most and holds their slots, coefficients and values in
+// registers for the whole launch; a step reads all sources, waits, and writes all
+// slots (a slot may be another link's source where the region wraps around a small
+// box).  Reading each table entry from memory in its cell, every step, one direction
+// after the other, made the launch as slow as the tile with most of them (per step,
+// entries in the cells / in the list: 901 x 219 channel around a cylinder,
+// interpolated walls, FP32 deviations 5.8 / 3.4 us; with plain walls, 1024 x 256 FP32
+// 3.8 / 3.5 us; 5000-cell 1D shock tube FP64 1.4 / 0.77 us).
+// A region with more links than the list holds takes the mask, table bits and first
+// entries of its cells into LDS and substitutes link by link in the cell.
 template <typename C>
 struct TbArgs {
   int32_t nt, tm, ti, tiles_i;
@@ -1051,9 +1067,19 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   constexpr int RC = tb_plane<S>();   // plane stride (cells), RN <= RC
   S* cur = reinterpret_cast<S*>(tb_smem);
   S* nxt = cur + NS * RC;
-  // constant over the launch: the region's mask words (folded links) and, with
-  // table links, every region cell's table bits and first entry (loaded with the
-  // populations, so a step reads its entries after one round trip instead of two)
+  // the link list lives in nxt until the first step; dense regions keep their mask
+  // words and, with table links, every cell's table bits and first entry after it
+  constexpr int LIST_AT = (NS * RC * (int)sizeof(S) + 31) / 16 * 16;   // bytes, counter 16 before
+  constexpr int LIST_FIT = (2 * NS * RC * (int)sizeof(S) - LIST_AT) / 8;
+  int* nlinks = reinterpret_cast<int*>(reinterpret_cast<char*>(tb_smem) + LIST_AT - 16);
+  uint2* links = reinterpret_cast<uint2*>(reinterpret_cast<char*>(tb_smem) + LIST_AT);
+  const bool masked = TB_MASK && a.bbmask;
+  const int cap = min(LIST_FIT, TB_LINKS * (int)blockDim.x);
+  (void)nlinks; (void)links; (void)cap;
+  if (masked) {
+    if (threadIdx.x == 0) *nlinks = 0;
+    __syncthreads();
+  }
   uint32_t* msk = reinterpret_cast<uint32_t*>(cur + 2 * NS * RC);
   uint32_t* tbits = msk + RN;
   uint32_t* tbase_l = tbits + RN;
@@ -1073,17 +1099,12 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
     const int64_t src = (int64_t)(a.halo[0] * a.n1 + gm + a.halo[1]) * a.rs + a.lead + gi + a.halo[2];
 #pragma unroll
     for (int k = 0; k < NS; ++k) cur[k * RC + c] = f[a.dst_off[k] + src];
-    if (TB_MASK && a.bbmask) {
-      const int64_t mc = (int64_t)gm * a.nin[2] + gi;
-      msk[c] = a.bbmask[mc];
-      if (table) {
-        tbits[c] = a.bbtab_bits[mc];
-        tbase_l[c] = a.bbtab_base[mc];
-      }
-    }
+%(tb_collect)s
   }
   __syncthreads();
+%(tb_entries)s
   for (int s = 1; s <= t.nt; ++s) {
+%(tb_apply)s
     const C tt = t.times[s - 1];
     (void)tt;
     const int WC = RI - 2 * s, HC = RW - 2 * s * MH;
@@ -1374,12 +1395,108 @@ def generate_source(spec: KernelSpec) -> str:
         tb_loads = ["S %s;" % ", ".join("L%d[1]" % k for k in range(ns))]
         tb_loads += ["L%d[0] = cur[%d * RC + lcell - (%d * RI + %d)];" % (k, k, vel[k][1], vel[k][2])
                      for k in range(ns)]
-        tb_sub = []
+        tb_sub, tb_collect, tb_entries, tb_apply = [], [], [], []
         if ksym is not None:
-            # bounce-back copies as selects of unconditional LDS reads (one branch per
+            # the links of every cell that the region updates (all but its outermost
+            # cells), listed as {slot | cell << 16, source} or, for a table entry,
+            # {slot | cell << 16, 1 << 31 | entry}
+            inner = "c - lr * RI > 0 && c - lr * RI < RI - 1" + (" && lr > 0 && lr < RW - 1" if dim == 2 else "")
+            tb_collect = ["if (masked && %s) {" % inner,
+                          "  const int64_t mc = (int64_t)gm * a.nin[2] + gi;",
+                          "  const uint32_t bits = a.bbmask[mc];",
+                          "  if (bits) {",
+                          "    const uint32_t tb = (bits & 0x80000000u) ? a.bbtab_bits[mc] : 0u;",
+                          "    const uint32_t tbase = tb ? a.bbtab_base[mc] : 0u;",
+                          "    int p_ = atomicAdd(nlinks, __builtin_popcount(bits & %du));"
+                          % sum(1 << k for k in range(ns) if ksym[k] != k)]
+            for k in range(ns):
+                if ksym[k] != k:
+                    bit = 1 << k
+                    tb_collect += ["    if (bits & %du) {" % bit,
+                                   "      if (p_ < cap)",
+                                   "        links[p_] = make_uint2((uint32_t)(%d * RC + c - (%d * RI + %d)) | ((uint32_t)c << 16),"
+                                   % (k, vel[k][1], vel[k][2]),
+                                   "                               (tb & %du) ? 0x80000000u | (tbase + (uint32_t)__builtin_popcount(tb & %du))"
+                                   % (bit, bit - 1),
+                                   "                                          : (uint32_t)(%d * RC + c));" % ksym[k],
+                                   "      ++p_;",
+                                   "    }"]
+            tb_collect += ["  }", "}"]
+            # this thread's links in registers: slot and source (16 bits each), second
+            # source, kind (0: none, 1: a copy, 2: one source, 3: two), coefficients, value
+            tb_entries = ["const int nlist = masked ? *nlinks : 0;",
+                          "const bool dense = nlist > cap;",
+                          "uint32_t l_at[TB_LINKS], l_two[TB_LINKS];",
+                          "C l_a[TB_LINKS], l_b[TB_LINKS], l_r[TB_LINKS];",
+                          "#pragma unroll",
+                          "for (int q = 0; q < TB_LINKS; ++q) {",
+                          "  const int e = q * (int)blockDim.x + (int)threadIdx.x;",
+                          "  l_at[q] = l_two[q] = 0;",
+                          "  l_a[q] = l_b[q] = l_r[q] = (C)0;",
+                          "  if (e < nlist && !dense) {",
+                          "    const uint2 w = links[e];",
+                          "    if (w.y & 0x80000000u) {",
+                          "      const uint32_t x = w.y & 0x7fffffffu;",
+                          "      const uint32_t rel = a.bbtab_rel[x];",
+                          "      const uint32_t rel2 = a.bbtab_rel2 ? a.bbtab_rel2[x] : 0u;",
+                          "      l_a[q] = a.bbtab_sign[x];",
+                          "      l_r[q] = a.bbtab_rhs[x];",
+                          "      l_b[q] = a.bbtab_rel2 ? a.bbtab_c2[x] : (C)0;",
+                          "      const int c = (int)(w.x >> 16);",
+                          "      const int src = (int)(rel & 0xffu) * RC + c + ((int)((rel >> 8) & 0xffu) - 128) * RI +",
+                          "                      (int)((rel >> 16) & 0xffu) - 128;",
+                          "      const int src2 = (int)(rel2 & 0xffu) * RC + c + ((int)((rel2 >> 8) & 0xffu) - 128) * RI +",
+                          "                       (int)((rel2 >> 16) & 0xffu) - 128;",
+                          "      const bool two = (rel2 & 0x80000000u) != 0;",
+                          "      l_at[q] = (w.x & 0xffffu) | ((uint32_t)src << 16);",
+                          "      l_two[q] = two ? 3u | ((uint32_t)src2 << 16) : 2u;",
+                          "    } else {",
+                          "      l_at[q] = (w.x & 0xffffu) | (w.y << 16);",
+                          "      l_two[q] = 1u;",
+                          "    }",
+                          "  }",
+                          "}",
+                          "__syncthreads();   // the list is read: nxt is free",
+                          "if (dense) {",
+                          "  for (int c = threadIdx.x; c < RN; c += blockDim.x) {",
+                          "    const int lr = c / RI;",
+                          "    const int gm = wrap_near(m0 + lr, a.nin[1]), gi = wrap_near(i0 + c - lr * RI, a.nin[2]);",
+                          "    const int64_t mc = (int64_t)gm * a.nin[2] + gi;",
+                          "    msk[c] = a.bbmask[mc];",
+                          "    if (table) {",
+                          "      tbits[c] = a.bbtab_bits[mc];",
+                          "      tbase_l[c] = a.bbtab_base[mc];",
+                          "    }",
+                          "  }",
+                          "  __syncthreads();",
+                          "}"]
+            # the arithmetic of fused_step's table entries (products and sums round apart)
+            tb_apply = ["if (nlist && !dense) {",
+                        "  S l_v[TB_LINKS];",
+                        "#pragma unroll",
+                        "  for (int q = 0; q < TB_LINKS; ++q) {",
+                        "    if (l_two[q]) {",
+                        "      const S v = cur[l_at[q] >> 16];",
+                        "      l_v[q] = v;",
+                        "      if (l_two[q] != 1u) {",
+                        "        C r_ = l_a[q] * Codec<S>::decode_dev(v, (C)0);",
+                        "        if ((l_two[q] & 0xffffu) == 3u)",
+                        "          r_ = r_ + l_b[q] * Codec<S>::decode_dev(cur[l_two[q] >> 16], (C)0);",
+                        "        r_ += l_r[q];",
+                        "        l_v[q] = Codec<S>::encode(r_, (C)0);",
+                        "      }",
+                        "    }",
+                        "  }",
+                        "  __syncthreads();",
+                        "#pragma unroll",
+                        "  for (int q = 0; q < TB_LINKS; ++q)",
+                        "    if (l_two[q]) cur[l_at[q] & 0xffffu] = l_v[q];",
+                        "  __syncthreads();",
+                        "}"]
+            # dense regions: bounce-back copies as selects of unconditional LDS reads (one branch per
             # cell instead of one per direction), then the table links: bits and
             # first entry from LDS, the entries from memory
-            tb_sub = ["if (a.bbmask) {",
+            tb_sub = ["if (dense) {",
                       "  const uint32_t bits = msk[lcell];",
                       "  if (bits) {"]
             for k in range(ns):
@@ -1425,6 +1542,7 @@ def generate_source(spec: KernelSpec) -> str:
                 tb_sub += ["      }"]
             tb_sub += ["    }", "  }", "}"]
         tb_kernel = _TB_KERNEL % dict(
+            tb_collect=_indent(tb_collect, 4), tb_entries=_indent(tb_entries), tb_apply=_indent(tb_apply, 4),
             tb_loads=_indent(tb_loads, 6), tb_sub=_indent(tb_sub, 6),
             tb_gdecl=_indent(["S %s;" % ", ".join("G%d[1]" % k for k in range(ns))], 6),
             tb_coords=_indent(coords, 6), tb_decode=_indent(decode, 6), tb_f2m=_indent(f2m_block, 6),

@@ -33,3 +33,29 @@ def test_1d_periodic_and_walls(hip, n, dtype):
 @pytest.mark.parametrize("n", [40, 777])
 def test_1d_shock_tube(hip, n):
     _equal(lambda: demos.riemann_euler(1.0 / n)[0], "float64", (130,))
+
+
+def _stripes(n, valued):
+    """Fluid columns one cell wide between solid ones: three links per cell, more than
+    the link list of a region holds (every wall carries the lid's value when valued)."""
+    from pylbm_amd.elements import Parallelogram
+    d = cases.lid_cavity_d2q9(n)
+    d["elements"] = [Parallelogram((x - 0.25, -1.0), (0.5, 0.0), (0.0, n + 2.0), label=1 if valued else 0)
+                     for x in np.arange(0.5, n, 2.0)]
+    return d
+
+
+# regions with more links than their list holds, with and without table entries, and
+# lists longer than one link per thread (every wall of a small box, wrapped many times
+# into the region)
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+def test_2d_dense_and_long_link_lists(hip, dtype):
+    for valued in (False, True):
+        _equal(lambda: _stripes(48, valued), dtype, (9,))
+
+    def small():
+        d = cases.lid_cavity_d2q9(9)
+        d["box"]["label"] = [1, 1, 1, 1]
+        return d
+    _equal(small, dtype, (13,))
+    _equal(lambda: cases.with_bouzidi(cases.karman_d2q9(90, 50, radius=9.3, center=(25.2, 24.7))), dtype, (14,))
