@@ -429,6 +429,7 @@ using namespace lbm;
 #define TB_MAX_NT (DIM == 1 ? 64 : 16) // steps per temporally blocked launch, at most
 #define TB_PLANE_1D 256                // cells of a 1D region, at most
 #define TB_MASK %(bbsub_ok)d                    // folded links possible
+#define TB_BATCH 2                     // cells a thread of a blocked workgroup loads at once
 #define TB_LINKS 4                     // folded links a thread of a blocked workgroup holds
 
 namespace {
@@ -1030,6 +1031,7 @@ _TB_KERNEL = r"""// ------------------------------------------------ temporally 
 template <typename C>
 struct TbArgs {
   int32_t nt, tm, ti, tiles_i;
+  uint32_t inv_ti, inv[TB_MAX_NT + 1];   // reciprocals of ti and of the row length after each step
   C times[TB_MAX_NT];   // t of each step (the host's sequence of t += dt)
 };
 
@@ -1042,20 +1044,29 @@ __device__ __forceinline__ int wrap_near(int x, int n) {
   return x;
 }
 
+// c / w for 0 <= c, w < 2^16 with inv = reciprocal(w): a 32-bit division is some 35
+// instructions, and every thread needs one per step to find its cells
+inline uint32_t reciprocal(int w) { return w > 1 ? (uint32_t)(((uint64_t)1 << 32) / w + 1) : 0u; }
+__device__ __forceinline__ int divide(int c, uint32_t inv) {
+  return inv ? (int)__umulhi((unsigned)c, inv) : c;
+}
+
 // Population planes of the region lie TB_PLANE<S> cells apart: a compile-time
 // stride, so that the plane offsets of the pulls and stores become immediates of
 // the LDS instructions.  It is the most cells the two copies of the populations
 // plus the mask / table words fit in 160 KiB with, and keeps the last plane within
 // the 16-bit immediate offset.
-template <typename S>
+// With HALF a workgroup takes half the LDS and two share a CU: one loads or stores
+// while the other computes.
+template <typename S, bool HALF>
 __host__ __device__ constexpr int tb_plane() {
   if (DIM == 1) return TB_PLANE_1D;
-  constexpr int a = (160 * 1024) / (2 * NS * (int)sizeof(S) + 12);
+  constexpr int a = ((HALF ? 80 : 160) * 1024) / (2 * NS * (int)sizeof(S) + 12);
   constexpr int b = NS > 1 ? 65528 / ((NS - 1) * (int)sizeof(S)) : a;
   return a < b ? a : b;
 }
 
-template <typename S>
+template <typename S, bool HALF>
 __global__ void __launch_bounds__(TB_THREADS)
 tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Codec<S>::C> a,
         const TbArgs<typename Codec<S>::C> t) {
@@ -1064,7 +1075,7 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   extern __shared__ uint4 tb_smem[];
   constexpr int MH = DIM == 2;   // the mid axis has a halo (a 1D region is one row)
   const int RW = t.tm + 2 * t.nt * MH, RI = t.ti + 2 * t.nt, RN = RW * RI;
-  constexpr int RC = tb_plane<S>();   // plane stride (cells), RN <= RC
+  constexpr int RC = tb_plane<S, HALF>();   // plane stride (cells), RN <= RC
   S* cur = reinterpret_cast<S*>(tb_smem);
   S* nxt = cur + NS * RC;
   // the link list lives in nxt until the first step; dense regions keep their mask
@@ -1093,13 +1104,33 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   const C* omega = a.omega;
   const C* cref = a.cref;
   (void)cref;
-  for (int c = threadIdx.x; c < RN; c += blockDim.x) {
-    const int lr = c / RI;
-    const int gm = wrap_near(m0 + lr, a.nin[1]), gi = wrap_near(i0 + c - lr * RI, a.nin[2]);
-    const int64_t src = (int64_t)(a.halo[0] * a.n1 + gm + a.halo[1]) * a.rs + a.lead + gi + a.halo[2];
+  // TB_BATCH cells per thread in flight: all their loads are issued before the first
+  // is written to LDS
+  for (int c0 = threadIdx.x; c0 < RN; c0 += TB_BATCH * blockDim.x) {
+    S v[TB_BATCH][NS];
+    uint32_t bits_[TB_BATCH];
 #pragma unroll
-    for (int k = 0; k < NS; ++k) cur[k * RC + c] = f[a.dst_off[k] + src];
+    for (int b = 0; b < TB_BATCH; ++b) {
+      const int c = c0 + b * (int)blockDim.x;
+      bits_[b] = 0;
+      if (c < RN) {
+        const int lr = divide(c, t.inv[0]);
+        const int gm = wrap_near(m0 + lr, a.nin[1]), gi = wrap_near(i0 + c - lr * RI, a.nin[2]);
+        const int64_t src = (int64_t)(a.halo[0] * a.n1 + gm + a.halo[1]) * a.rs + a.lead + gi + a.halo[2];
+%(tb_mask)s
+#pragma unroll
+        for (int k = 0; k < NS; ++k) v[b][k] = f[a.dst_off[k] + src];
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < TB_BATCH; ++b) {
+      const int c = c0 + b * (int)blockDim.x;
+      if (c < RN) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) cur[k * RC + c] = v[b][k];
+      }
 %(tb_collect)s
+    }
   }
   __syncthreads();
 %(tb_entries)s
@@ -1111,8 +1142,8 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
     // the cells of the shrunk region in row-major order, blockDim.x apart: the
     // (row, column) of the next one follow by adding (dq, dr) with a carry, and its
     // region index by adding dl, plus dc on a carry (no multiply per cell)
-    const int dq = (int)blockDim.x / WC, dr = (int)blockDim.x - dq * WC;
-    int rr = (int)threadIdx.x / WC, qq = (int)threadIdx.x - rr * WC;
+    const int dq = divide((int)blockDim.x, t.inv[s]), dr = (int)blockDim.x - dq * WC;
+    int rr = divide((int)threadIdx.x, t.inv[s]), qq = (int)threadIdx.x - rr * WC;
     const int dl = dq * RI + dr, dc = RI - WC;
     int lnext = (s * MH + rr) * RI + s + qq;
     for (int c = threadIdx.x; c < WC * HC; c += blockDim.x) {
@@ -1155,7 +1186,8 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
     nxt = tmp;
   }
   for (int c = threadIdx.x; c < t.tm * t.ti; c += blockDim.x) {
-    const int lr = t.nt * MH + c / t.ti, lc = t.nt + c %% t.ti;
+    const int q = divide(c, t.inv_ti);
+    const int lr = t.nt * MH + q, lc = t.nt + c - q * t.ti;
     const int gm = m0 + lr, gi = i0 + lc;
     if (gm >= a.nin[1] || gi >= a.nin[2]) continue;
     const int64_t dst = (int64_t)(a.halo[0] * a.n1 + gm + a.halo[1]) * a.rs + a.lead + gi + a.halo[2];
@@ -1181,22 +1213,30 @@ static int tb_launch(void* f, void* fn, const lbm_layout* L, lbm_params* p, int 
   t.tm = tm;
   t.ti = ti;
   t.tiles_i = (a.nin[2] + ti - 1) / ti;
+  t.inv_ti = reciprocal(ti);
+  for (int q = 0; q <= nt; ++q) t.inv[q] = reciprocal(ti + 2 * (nt - q));
   for (int q = 0; q < nt; ++q) {
     t.times[q] = (C)p->t;
     p->t += p->dt;
   }
   const int tiles_m = (a.nin[1] + tm - 1) / tm;
   const size_t region = (size_t)(DIM == 1 ? tm : tm + 2 * nt) * (ti + 2 * nt);
-  // a thread per region cell, at most TB_THREADS: a 1D region needs few waves
-  const unsigned threads = DIM == 1 ? (unsigned)((region + 63) / 64 * 64) : TB_THREADS;
   const bool mask = TB_MASK && p->bbmask, table = mask && p->bbtab_bits;
-  LBM_REQUIRE(region <= (size_t)tb_plane<S>(), "tile region of %%zu cells exceeds the %%d cells of a plane",
-              region, tb_plane<S>());
-  const size_t lds = 2 * NS * sizeof(S) * (size_t)tb_plane<S>() + region * ((mask ? 4 : 0) + (table ? 8 : 0));
+  constexpr size_t full_plane = tb_plane<S, false>(), half_plane = tb_plane<S, true>();
+  LBM_REQUIRE(region <= full_plane, "tile region of %%zu cells exceeds the %%zu cells of a plane", region, full_plane);
+  const bool half = region <= half_plane;
+  const size_t plane = half ? half_plane : full_plane;
+  const size_t lds = 2 * NS * sizeof(S) * plane + region * ((mask ? 4 : 0) + (table ? 8 : 0));
   LBM_REQUIRE(lds <= 160 * 1024, "tile needs %%zu bytes of LDS", lds);
-  LBM_CHECK_HIP(hipFuncSetAttribute((const void*)tb_step<S>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds));
-  tb_step<S><<<dim3((unsigned)(tiles_m * t.tiles_i)), dim3(threads), lds, s>>>((const S*)f, (S*)fn, a, t);
+  // a thread per region cell, at most TB_THREADS, or half as many where two
+  // workgroups share a CU
+  const unsigned tiles = (unsigned)(tiles_m * t.tiles_i);
+  const unsigned most = half && tiles > 256 ? TB_THREADS / 2 : TB_THREADS;
+  const unsigned threads = (unsigned)(region < most ? (region + 63) / 64 * 64 : most);
+  const void* kernel = half ? (const void*)tb_step<S, true> : (const void*)tb_step<S, false>;
+  LBM_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  if (half) tb_step<S, true><<<dim3(tiles), dim3(threads), lds, s>>>((const S*)f, (S*)fn, a, t);
+  else tb_step<S, false><<<dim3(tiles), dim3(threads), lds, s>>>((const S*)f, (S*)fn, a, t);
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1395,16 +1435,18 @@ def generate_source(spec: KernelSpec) -> str:
         tb_loads = ["S %s;" % ", ".join("L%d[1]" % k for k in range(ns))]
         tb_loads += ["L%d[0] = cur[%d * RC + lcell - (%d * RI + %d)];" % (k, k, vel[k][1], vel[k][2])
                      for k in range(ns)]
-        tb_sub, tb_collect, tb_entries, tb_apply = [], [], [], []
+        tb_sub, tb_mask, tb_collect, tb_entries, tb_apply = [], [], [], [], []
         if ksym is not None:
             # the links of every cell that the region updates (all but its outermost
             # cells), listed as {slot | cell << 16, source} or, for a table entry,
             # {slot | cell << 16, 1 << 31 | entry}
             inner = "c - lr * RI > 0 && c - lr * RI < RI - 1" + (" && lr > 0 && lr < RW - 1" if dim == 2 else "")
-            tb_collect = ["if (masked && %s) {" % inner,
-                          "  const int64_t mc = (int64_t)gm * a.nin[2] + gi;",
-                          "  const uint32_t bits = a.bbmask[mc];",
+            tb_mask = ["if (masked && %s) bits_[b] = a.bbmask[(int64_t)gm * a.nin[2] + gi];" % inner]
+            tb_collect = ["{",
+                          "  const uint32_t bits = bits_[b];",
                           "  if (bits) {",
+                          "    const int lr = divide(c, t.inv[0]);",
+                          "    const int64_t mc = (int64_t)wrap_near(m0 + lr, a.nin[1]) * a.nin[2] + wrap_near(i0 + c - lr * RI, a.nin[2]);",
                           "    const uint32_t tb = (bits & 0x80000000u) ? a.bbtab_bits[mc] : 0u;",
                           "    const uint32_t tbase = tb ? a.bbtab_base[mc] : 0u;",
                           "    int p_ = atomicAdd(nlinks, __builtin_popcount(bits & %du));"
@@ -1459,7 +1501,7 @@ def generate_source(spec: KernelSpec) -> str:
                           "__syncthreads();   // the list is read: nxt is free",
                           "if (dense) {",
                           "  for (int c = threadIdx.x; c < RN; c += blockDim.x) {",
-                          "    const int lr = c / RI;",
+                          "    const int lr = divide(c, t.inv[0]);",
                           "    const int gm = wrap_near(m0 + lr, a.nin[1]), gi = wrap_near(i0 + c - lr * RI, a.nin[2]);",
                           "    const int64_t mc = (int64_t)gm * a.nin[2] + gi;",
                           "    msk[c] = a.bbmask[mc];",
@@ -1475,6 +1517,7 @@ def generate_source(spec: KernelSpec) -> str:
                         "  S l_v[TB_LINKS];",
                         "#pragma unroll",
                         "  for (int q = 0; q < TB_LINKS; ++q) {",
+                        "    if (q * (int)blockDim.x >= nlist) break;   // the same for the whole workgroup",
                         "    if (l_two[q]) {",
                         "      const S v = cur[l_at[q] >> 16];",
                         "      l_v[q] = v;",
@@ -1489,8 +1532,10 @@ def generate_source(spec: KernelSpec) -> str:
                         "  }",
                         "  __syncthreads();",
                         "#pragma unroll",
-                        "  for (int q = 0; q < TB_LINKS; ++q)",
+                        "  for (int q = 0; q < TB_LINKS; ++q) {",
+                        "    if (q * (int)blockDim.x >= nlist) break;",
                         "    if (l_two[q]) cur[l_at[q] & 0xffffu] = l_v[q];",
+                        "  }",
                         "  __syncthreads();",
                         "}"]
             # dense regions: bounce-back copies as selects of unconditional LDS reads (one branch per
@@ -1542,7 +1587,7 @@ def generate_source(spec: KernelSpec) -> str:
                 tb_sub += ["      }"]
             tb_sub += ["    }", "  }", "}"]
         tb_kernel = _TB_KERNEL % dict(
-            tb_collect=_indent(tb_collect, 4), tb_entries=_indent(tb_entries), tb_apply=_indent(tb_apply, 4),
+            tb_mask=_indent(tb_mask, 8), tb_collect=_indent(tb_collect, 6), tb_entries=_indent(tb_entries), tb_apply=_indent(tb_apply, 4),
             tb_loads=_indent(tb_loads, 6), tb_sub=_indent(tb_sub, 6),
             tb_gdecl=_indent(["S %s;" % ", ".join("G%d[1]" % k for k in range(ns))], 6),
             tb_coords=_indent(coords, 6), tb_decode=_indent(decode, 6), tb_f2m=_indent(f2m_block, 6),

@@ -18,6 +18,7 @@ FP32 / FP16 / BF16; every non-FP64 format computes the collision in FP32 on
 deviations from the rest state); ``conserved_sums()`` returns FP64 compensated global sums.
 """
 import ctypes
+import functools
 import math
 import time
 import types
@@ -51,6 +52,59 @@ FOLD_TABLE_MAX = 1 << 16
 # and 0.77 us this way.
 TB_SHAPE_1D = (64, 128)
 TB_PLANE_1D = 256
+
+
+@functools.lru_cache(maxsize=256)
+def _blocked_tile(ns, es, n0, n1, links):
+    """(steps per launch, tile rows, tile columns) of the temporally blocked 2D run of a
+    scheme of ns populations of es bytes on n0 x n1 cells, with folded links or
+    without; None when no tile fits the LDS or one launch per step is as fast.
+
+    A workgroup keeps two copies of its tile and a halo of steps cells in LDS: many
+    steps per launch share the launch and the load but recompute the halo, small tiles
+    fill the GPU but have more halo, two workgroups share a CU when a region fits half
+    its LDS.  The tile is the one whose estimated time per step is the least of
+    steps 2-12 x rows 4-48 x columns 8-64.  The estimate (us per launch; a sweep of
+    those tiles on MI355X over 64^2 to 3000 x 2800 cells in 8-, 4- and 2-byte formats,
+    D2Q9 and D2Q9 + D2Q5, with and without links, fitted its constants; the tiles it
+    picks take 2 % longer than the best measured ones on average, 11 % at most):
+      3.5 + 1.5 with links  launch, last store, building the link list
+      rounds x              tiles / 256, rounded up below 2048 tiles, x 3/4 where
+                            two tiles share a CU
+        0.103 per KB of region loaded, 0.15 (+ 0.29 with links) per step,
+        ns / 9 x (0.07, 0.10, 0.17 for 8, 4, 2 bytes) x (waves of cells / 4) per step.
+    Measured per step, one launch each / fixed tiles of 32 x 32 (FP64 16 x 32) / these:
+    3000 x 2800 FP32 107 / 68 / 63 us, FP64 216 / - / 137 us; 512^2 FP32 6.1 / 2.7 / 2.7 us;
+    128^2 FP64 lid cavity 4.7 / 2.8 / 1.7 us.  Past 2^21 cells (the caches no longer
+    hold them) the estimate is compared with the traffic of single steps at 5.6 TB/s."""
+    plane = min((160 * 1024) // (2 * ns * es + 12), 65528 // ((ns - 1) * es) if ns > 1 else 1 << 30)
+    half = min((80 * 1024) // (2 * ns * es + 12), plane)
+    per_wave = ns / 9.0 * {8: 0.07, 4: 0.10, 2: 0.17}[es]
+    best = None
+    for nt in (2, 3, 4, 5, 6, 7, 8, 10, 12):
+        if nt > min(n0, n1):
+            break
+        for tm in {min(t, n0) for t in (4, 8, 12, 16, 20, 24, 32, 40, 48)}:
+            for ti in {min(t, n1) for t in (8, 16, 24, 32, 40, 48, 64)}:
+                region = (tm + 2 * nt) * (ti + 2 * nt)
+                if region > plane:
+                    continue
+                tiles = -(-n0 // tm) * -(-n1 // ti)
+                shared = region <= half and tiles > 256
+                rounds = tiles / 256.0
+                if tiles < 2048:
+                    rounds = 2 * math.ceil(tiles / 512.0) if shared else math.ceil(rounds)
+                if shared:
+                    rounds *= 0.75
+                waves = sum(-(-((tm + 2 * s) * (ti + 2 * s)) // 256) for s in range(nt))
+                us = 3.5 + 1.5 * links + rounds * (1.03e-4 * region * ns * es + nt * (0.15 + 0.29 * links)
+                                                   + per_wave * waves)
+                key = (us / nt, nt, tm, ti)
+                if best is None or key < best:
+                    best = key
+    if best is None or (n0 * n1 > 1 << 21 and best[0] >= n0 * n1 * 2.0 * ns * es / 5.6e6):
+        return None
+    return best[1:]
 
 
 def _canon_velocities(spec, box_label=None):
@@ -767,15 +821,8 @@ class Simulation:
     def _blocking_shape(self):
         """(steps per launch, tile rows, tile columns) of the temporally blocked run, or
         None: 1D and 2D schemes on the wrap path (periodic, or every list folded with
-        its table sources within one cell), in 2D on grids small enough that a step
-        does not fill the GPU (at most 2^21 cells).  The tile and its halo live in LDS: two
-        copies of ns populations per cell in planes of a fixed size (the most cells
-        that fit the 160 KiB of a CU with the mask and table words), and the region
-        has to fit one plane.  The preferred shapes were measured on MI355X
-        (D2Q9, 128^2 to 1024 x 256): 6 steps of 32 x 32 tiles for the 4- and 2-byte
-        formats, 4 steps of 16 x 32 tiles for FP64, 6 steps of 8 x 16 tiles for FP64
-        grids of at most 2^15 cells (more tiles than CUs matter more there than the
-        recomputed halo); larger schemes shrink the tile until it fits."""
+        its table sources within one cell) with velocity components in {-1, 0, 1}.
+        The tile and its halo live in LDS (_blocked_tile)."""
         if not self.temporal_blocking or self.dim > 2 or not self._wrap:
             return None
         if np.any(np.abs(np.asarray(self.scheme.stencil.get_all_velocities())) > 1):
@@ -784,37 +831,14 @@ class Simulation:
                                                                       not self.params.bbtab_rel2):
             return None
         nin = [int(x) for x in self.domain.shape_in]
+        es = self.container.F.layout.elem_size
         if self.dim == 1:
             nt, ti = TB_SHAPE_1D
-            if 2 * self.ns * TB_PLANE_1D * self.container.F.layout.elem_size + 12 * TB_PLANE_1D > 160 * 1024:
+            if 2 * self.ns * TB_PLANE_1D * es + 12 * TB_PLANE_1D > 160 * 1024:
                 return None
             nt = min(nt, nin[0])
             return (nt, 1, min(ti, nin[0])) if nt >= 2 else None
-        cells = nin[0] * nin[1]
-        if cells > (1 << 21):
-            return None
-        es = self.container.F.layout.elem_size
-        # the kernel's population planes hold this many cells (tb_plane in the
-        # generated module): every region has to fit one plane
-        plane = min((160 * 1024) // (2 * self.ns * es + 12),
-                    65528 // ((self.ns - 1) * es) if self.ns > 1 else 1 << 30)
-        if es == 8:
-            nt, tm, ti = (6, 8, 16) if cells <= (1 << 15) else (4, 16, 32)
-        else:
-            nt, tm, ti = 6, 32, 32
-        while (tm + 2 * nt) * (ti + 2 * nt) > plane:
-            if ti > 16:
-                ti //= 2
-            elif tm > 8:
-                tm //= 2
-            elif nt > 2:
-                nt -= 1
-            else:
-                return None
-        nt = min(nt, min(nin))
-        if nt < 2:
-            return None
-        return nt, min(tm, nin[0]), min(ti, nin[1])
+        return _blocked_tile(self.ns, es, nin[0], nin[1], bool(self.params.bbmask))
 
     def sync(self):
         self.rt.sync()

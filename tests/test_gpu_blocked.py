@@ -59,3 +59,11 @@ def test_2d_dense_and_long_link_lists(hip, dtype):
         return d
     _equal(small, dtype, (13,))
     _equal(lambda: cases.with_bouzidi(cases.karman_d2q9(90, 50, radius=9.3, center=(25.2, 24.7))), dtype, (14,))
+
+
+# ragged 2D boxes: tiles and regions that do not divide them, boxes thinner than a tile,
+# and (more than 256 tiles in half planes) two workgroups per CU
+@pytest.mark.parametrize("dtype", ["float64", "float32", "bfloat16"])
+@pytest.mark.parametrize("nx,ny", [(4, 300), (301, 5), (37, 41), (700, 611)])
+def test_2d_ragged(hip, nx, ny, dtype):
+    _equal(lambda: cases.forced_periodic_d2q9(nx=nx, ny=ny, g0=1e-7), dtype, (25, 2))
