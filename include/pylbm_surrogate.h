@@ -92,7 +92,7 @@ typedef struct lbm_sur_net {
 int lbm_sur_run(lbm_sur_net* net, const float* d_src, float* d_state, const float* dscale, const float* shift,
                 const float* scale, int64_t nsteps, int N, int H, int W, void* stream);
 
-/* number of workgroups per tap (partial sums) lbm_sur_wgrad uses */
+/* number of partial sums lbm_sur_wgrad uses, at most */
 int lbm_sur_wgrad_blocks(void);
 
 /*
@@ -126,6 +126,28 @@ int lbm_sur_pack(const float* d_w, int cin, int cout, int cinp, int coutp, void*
  * (layout [9][coutp][cinp]) */
 int lbm_sur_adam(float* d_w, float* d_b, float* d_m, float* d_v, const float* d_dwt, const float* d_db, int cin,
                  int cout, int cinp, int coutp, float lr, float b1, float b2, float eps, int step, void* stream);
+
+/* the buffers of one layer for lbm_sur_adam_net: master weights and bias, their Adam
+ * moments and gradients as for lbm_sur_adam, operands as for lbm_sur_pack (abwd may be
+ * NULL) with cinp = cin, coutp = cout */
+#define LBM_SUR_MAX_LAYERS 4
+typedef struct lbm_sur_layer {
+  float* w;
+  float* b;
+  float* m;
+  float* v;
+  const float* dwt;
+  const float* db;
+  void* afwd;
+  void* abwd;
+  int32_t cin;
+  int32_t cout;
+} lbm_sur_layer;
+
+/* lbm_sur_adam and lbm_sur_pack of up to LBM_SUR_MAX_LAYERS layers in one launch (the
+ * same values) */
+int lbm_sur_adam_net(const lbm_sur_layer* layers, int nlayers, float lr, float b1, float b2, float eps, int step,
+                     int elem, void* stream);
 
 /* network input (E coarse [N][Hf/4][Wf/4][64]) = (state - shift) / scale per field
  * (3 host floats each) */

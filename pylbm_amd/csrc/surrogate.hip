@@ -58,8 +58,9 @@ constexpr int EPI_LIN = 1;    // y = acc + b as FP32
 constexpr int EPI_BWD = 2;    // g = acc * silu'(z_in): store E
 constexpr int EPI_APPLY = 3;  // fine state += (acc + b) * dscale, next network input
 
-constexpr int WG_PIX = 32;             // pixels per weight-gradient block iteration
-constexpr int SUR_WGRAD_BLOCKS = 64;   // weight-gradient workgroups per tap
+constexpr int WG_PIX = 32;             // pixels of one weight-gradient K step
+constexpr int WG_SEG = 64;             // pixels of a weight-gradient row segment
+constexpr int SUR_WGRAD_BLOCKS = 256;  // weight-gradient workgroups, at most: one per CU
 
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
 
@@ -99,17 +100,37 @@ struct ApplyArgs {
 };
 
 // ---------------------------------------------------------------- conv 3x3
-// Workgroup = 4 waves = one row segment of 64 pixels (4 tiles of 16, one per wave)
-// for all COUTP output channels.  The workgroup stages in LDS its input rows
-// y - 1 .. y + 1 over pixels x0 - 1 .. x0 + 64 (periodic wrap) and all weight rows;
-// both are padded by 16 bytes per pixel / row so that the 16 rows (pixels) one
-// MFMA operand read touches fall in distinct banks.  Then each wave runs its
-// 9 * CINP / 32 K steps of MT = COUTP / 16 independent MFMA chains from LDS.
+// Workgroup = 4 waves = a strip of `rows` rows of one 64-pixel segment (4 tiles of 16,
+// one per wave) for all COUTP output channels.  Input rows pass through a ring of four
+// LDS rows (pixels x0 - 1 .. x0 + 64, periodic wrap), the next one loaded while this
+// one's MFMAs run: one barrier per row.  The weights are read once per strip: into
+// registers where they fit (up to 36 operands of 16 x 32, conv_in_registers), else into
+// LDS.  Pixels and weight rows are padded by 16 bytes so that the 16 rows (pixels) one
+// MFMA operand read touches fall in distinct banks.  Each wave runs its 9 * CINP / 32 K
+// steps of MT = COUTP / 16 independent MFMA chains, tap by tap.
+// Bound by latency and the bytes of its activations (8 x 128 x 128 pixels: 25-33 MB, 4-6
+// us of traffic).  64 -> 32 channels 17 us, 32 -> 32 12 us, 32 -> 64 (FP32 out) 16 us;
+// a workgroup per row, its weights staged in LDS again for each, took 26, 14 and 21.
+template <int CINP, int COUTP>
+constexpr bool conv_in_registers() {
+  return COUTP / 16 * 9 * (CINP / 32) <= 36;
+}
+constexpr int CONV_SEG = 64, CONV_SPAN = CONV_SEG + 2;
+// rows of a strip: as many as leave CONV_GROUPS workgroups, at most CONV_ROWS (8 x 128 x
+// 128 pixels, training step: 256 / 512 / 1024 workgroups 223 / 203 / 224 us)
+constexpr int CONV_GROUPS = 512, CONV_ROWS = 8;
+
+template <int CINP, int COUTP>
+constexpr size_t conv_lds() {
+  constexpr size_t weights = (size_t)COUTP * (9 * CINP + 8) * EB, ring = 4 * CONV_SPAN * (CINP + 8) * EB;
+  return conv_in_registers<CINP, COUTP>() ? (weights > ring ? weights : ring) : weights + ring;
+}
+
 template <typename E, int CINP, int COUTP, int EPI>
 __global__ void __launch_bounds__(256) conv3x3_kernel(const E* __restrict__ in, const E* __restrict__ wpk,
                                                       const float* __restrict__ bias,
                                                       const E* __restrict__ zin, void* __restrict__ out,
-                                                      E* __restrict__ zout, int N, int H, int W,
+                                                      E* __restrict__ zout, int H, int W, int rows, int strips,
                                                       ApplyArgs ap) {
   typedef typename Elem<E>::v4 half4;
   typedef typename Elem<E>::v8 half8;
@@ -118,53 +139,74 @@ __global__ void __launch_bounds__(256) conv3x3_kernel(const E* __restrict__ in, 
   constexpr int KPP = KP + 8;
   constexpr int KC = CINP / 32;
   constexpr int CIP = CINP + 8;
-  constexpr int SEG = 64, SPAN = SEG + 2;
+  constexpr int SPAN = CONV_SPAN;
+  constexpr bool WREG = conv_in_registers<CINP, COUTP>();
+  constexpr int NX = SPAN * (CINP / 8), PX = (NX + 255) / 256;   // 16-byte items of a row
   static_assert(CINP % 32 == 0 && COUTP % 16 == 0, "channel tiling");
   extern __shared__ uint4 smem_u4[];
   E* smem = reinterpret_cast<E*>(smem_u4);
-  E* sw = smem;                         // [COUTP][KPP]
-  E* sx = smem + COUTP * KPP;           // [3][SPAN][CIP]
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int segs = (W + SEG - 1) / SEG;
-  const int n = blockIdx.x / (H * segs);
-  const int y = (blockIdx.x / segs) % H;
-  const int xs = (blockIdx.x % segs) * SEG;
+  E* sx = smem;                         // [4][SPAN][CIP]
+  E* sw = WREG ? smem : smem + 4 * SPAN * CIP;   // [COUTP][KPP], before the ring where they go to registers
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int segs = (W + CONV_SEG - 1) / CONV_SEG;
+  const int n = blockIdx.x / (strips * segs);
+  const int y0 = (blockIdx.x / segs) % strips * rows;
+  const int xs = (blockIdx.x % segs) * CONV_SEG;
+  const int nrows = min(rows, H - y0);
   const int g = lane >> 4, r = lane & 15;
-  // stage weights and input rows
-  {
-    constexpr int NW8 = COUTP * (KP / 8);
-    constexpr int NX8 = 3 * SPAN * (CINP / 8);
-    const E* img = in + (int64_t)n * H * W * CINP;
-    staged_copy<NW8>(
-        [&](int e) {
-          half8 v;
-          __builtin_memcpy(&v, wpk + (e / (KP / 8)) * KP + (e % (KP / 8)) * 8, 16);
-          return v;
-        },
-        [&](int e, const half8& v) { __builtin_memcpy(sw + (e / (KP / 8)) * KPP + (e % (KP / 8)) * 8, &v, 16); });
-    staged_copy<NX8>(
-        [&](int f) {
-          const int c8 = (f % (CINP / 8)) * 8, q = (f / (CINP / 8)) % SPAN, dyi = f / ((CINP / 8) * SPAN);
-          // rows with W < 64 wrap more than once: full modulo
-          const int yy = wrap(y + dyi - 1, H), xx = (xs + q - 1 + W) % W;
-          half8 v;
-          __builtin_memcpy(&v, img + ((int64_t)yy * W + xx) * CINP + c8, 16);
-          return v;
-        },
-        [&](int f, const half8& v) {
-          const int c8 = (f % (CINP / 8)) * 8, q = (f / (CINP / 8)) % SPAN, dyi = f / ((CINP / 8) * SPAN);
-          __builtin_memcpy(sx + (dyi * SPAN + q) * CIP + c8, &v, 16);
-        });
-  }
-  __syncthreads();
   const int x0 = xs + wv * 16;
-  if (x0 >= W) return;
+  half8 wr[WREG ? MT : 1][WREG ? 9 * KC : 1];
+  const E* img = in + (int64_t)n * H * W * CINP;
+  const auto load_row = [&](int y, half8 (&vx)[PX]) {
+    const E* row = img + (int64_t)wrap(y, H) * W * CINP;
+#pragma unroll
+    for (int q = 0; q < PX; ++q) {
+      const int e = min(tid + q * 256, NX - 1);
+      const int xx = (xs + e / (CINP / 8) - 1 + W) % W;   // rows with W < 64 wrap more than once
+      vx[q] = *reinterpret_cast<const half8*>(row + (int64_t)xx * CINP + e % (CINP / 8) * 8);
+    }
+  };
+  const auto store_row = [&](int slot, const half8 (&vx)[PX]) {
+#pragma unroll
+    for (int q = 0; q < PX; ++q) {
+      const int e = tid + q * 256;
+      if (e < NX) *reinterpret_cast<half8*>(sx + (slot * SPAN + e / (CINP / 8)) * CIP + e % (CINP / 8) * 8) = vx[q];
+    }
+  };
+  // row y0 + j - 1 + i lies in ring slot i % 4
+  half8 v0[PX], v1[PX], v2[PX];
+  load_row(y0 - 1, v0);
+  load_row(y0, v1);
+  load_row(y0 + 1, v2);
+  staged_copy<COUTP * (KP / 8)>(
+      [&](int e) {
+        half8 v;
+        __builtin_memcpy(&v, wpk + (e / (KP / 8)) * KP + (e % (KP / 8)) * 8, 16);
+        return v;
+      },
+      [&](int e, const half8& v) { __builtin_memcpy(sw + (e / (KP / 8)) * KPP + (e % (KP / 8)) * 8, &v, 16); });
+  if constexpr (WREG) {
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int k = 0; k < 9 * KC; ++k) __builtin_memcpy(&wr[mt][k], sw + (mt * 16 + r) * KPP + k * 32 + g * 8, 16);
+    __syncthreads();
+  }
+  store_row(0, v0);
+  store_row(1, v1);
+  store_row(2, v2);
+  for (int j = 0; j < nrows; ++j) {
+  const int y = y0 + j;
+  if (j + 1 < nrows) load_row(y + 2, v0);
+  __syncthreads();
+  if (x0 < W) {
   float4v acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int t = 0; t < 9; ++t) {
-    const E* bx = sx + ((t / 3) * SPAN + wv * 16 + r + t % 3) * CIP + g * 8;
+    const E* bx = sx + ((j + t / 3 & 3) * SPAN + wv * 16 + r + t % 3) * CIP + g * 8;
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
       half8 b;
@@ -172,7 +214,8 @@ __global__ void __launch_bounds__(256) conv3x3_kernel(const E* __restrict__ in, 
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         half8 a;
-        __builtin_memcpy(&a, sw + (mt * 16 + r) * KPP + t * CINP + kc * 32 + g * 8, 16);
+        if constexpr (WREG) a = wr[mt][t * KC + kc];
+        else __builtin_memcpy(&a, sw + (mt * 16 + r) * KPP + t * CINP + kc * 32 + g * 8, 16);
         acc[mt] = Elem<E>::mfma(a, b, acc[mt]);
       }
     }
@@ -225,6 +268,9 @@ __global__ void __launch_bounds__(256) conv3x3_kernel(const E* __restrict__ in, 
       __builtin_memcpy(ap.state + fp * 4, &s, 16);
       __builtin_memcpy((E*)ap.xnext + p * 64 + c0, &xb, 8);
     }
+  }
+  }
+  if (j + 1 < nrows) store_row(j + 3 & 3, v0);
   }
 }
 
@@ -498,98 +544,179 @@ __global__ void __launch_bounds__(64 * FUSED_WAVES) fused_step_kernel(const E* _
   fused_layer<E, C, 3, C, 64>(bufB, nullptr, sw1, b3, n, y0, x0, H, W, ap);
 }
 
-// -------------------------------------------------------- weight gradient
-// Workgroup (bx, tap): partial sums of dW[tap]^T[co][ci] = sum_p dZ[p][co] X[p + d_tap][ci]
-// over the blocks of WG_PIX pixels bx, bx + gridDim.x, ...; the tap-4 (centre) row of
-// the grid also sums db[co] = sum_p dZ[p][co].
+// Weight and bias gradients: dW[tap]^T[co][ci] = sum over pixels p of dZ[p][co] X[p + d_tap][ci].
+// The pixels are the K dimension of the MFMA, so both operands are wanted with eight
+// pixels of one channel per lane while memory has the channels of one pixel together:
+// rows are staged in LDS as they lie in memory and read with ds_read_b64_tr_b16, which
+// hands lane i of 16 the values of channel i of four pixels.  A tap is then only another
+// first pixel, so one workgroup computes all nine taps from one read of dZ and X: it
+// walks down a strip of rows, 64 pixels wide, with the next row's loads in flight while
+// the MFMAs of this row run (X: a ring of four rows, dZ: two).  A wave keeps one input
+// tile of 16 channels and MT * NT / 4 output tiles, 9 accumulators each.
+// Bound by latency and the partial sums (8 x 128 x 128 pixels: the bytes take 4-6 us, the
+// MFMAs 1-2).  32 x 32 channels 13 us, 64 x 32 17 us, 32 x 64 19 us; one workgroup row
+// per tap, operands transposed on their way into LDS 16 bits at a time, took 48, 90 and 83.
+template <typename E>
+__device__ __forceinline__ typename Elem<E>::v8 read_tr(const E* base, int stride) {
+  // lane (g, i): pixels 8 g + [0, 8), channel i of the 16 at base (stride elements per pixel)
+  typedef short short4v __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) short4v* lds4;
+  const int g = (threadIdx.x & 63) >> 4, i = threadIdx.x & 15;
+  const E* p = base + (g * 8 + (i >> 2)) * stride + (i & 3) * 4;
+  const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p);
+  const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(p + 4 * stride));
+  typename Elem<E>::v8 v;
+  __builtin_memcpy(&v, &lo, 8);
+  __builtin_memcpy((char*)&v + 8, &hi, 8);
+  return v;
+}
+
 template <typename E, int CINP, int CDZ>
 __global__ void __launch_bounds__(256) conv3x3_wgrad_kernel(const E* __restrict__ x, const E* __restrict__ dz,
                                                             float* __restrict__ partial,
-                                                            float* __restrict__ partial_b, int N, int H, int W) {
-  typedef typename Elem<E>::v4 half4;
+                                                            float* __restrict__ partial_b, int H, int W, int rows,
+                                                            int strips, int tasks) {
   typedef typename Elem<E>::v8 half8;
-  constexpr int MT = CDZ / 16, NT = CINP / 16;
-  constexpr int TILES = MT * NT;
-  static_assert(TILES % 4 == 0, "tiles per wave");
-  constexpr int PER_WAVE = TILES / 4;
-  constexpr int LP = WG_PIX + 8;  // padded pixel stride of the transposed tiles (80 B)
-  __shared__ __attribute__((aligned(16))) E sdz[CDZ][LP];
-  __shared__ __attribute__((aligned(16))) E sx[CINP][LP];
-  const int tap = blockIdx.y;
-  const int dy = tap / 3 - 1, dx = tap % 3 - 1;
+  constexpr int NT = CINP / 16, PW = CDZ / 16 * NT / 4;   // output tiles per wave
+  constexpr int SPAN = WG_SEG + 2, XS = CINP + 8, ZS = CDZ + 8;   // padded pixels: 16 B apart in the banks
+  constexpr int NX = SPAN * (CINP / 8), NZ = WG_SEG * (CDZ / 8);   // 16-byte items of a row
+  constexpr int PX = (NX + 255) / 256, PZ = (NZ + 255) / 256;
+  __shared__ __attribute__((aligned(16))) E sx[4 * SPAN * XS];
+  __shared__ __attribute__((aligned(16))) E sz[2 * WG_SEG * ZS];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = lane >> 4, r = lane & 15;
-  float4v acc[PER_WAVE];
+  const int nt = wv % NT, mt0 = wv / NT * PW;
+  float4v acc[PW][9];
 #pragma unroll
-  for (int q = 0; q < PER_WAVE; ++q) acc[q] = float4v{0.f, 0.f, 0.f, 0.f};
-  float bacc = 0.f;  // bias partial of channel tid / 4 over pixels (tid % 4) * 8 + [0, 8)
-  const int segs = W / WG_PIX;
-  const int nblocks = N * H * segs;
-  for (int blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
-    const int n = blk / (H * segs), y = (blk / segs) % H, x0 = (blk % segs) * WG_PIX;
-    __syncthreads();
-    for (int e = tid; e < WG_PIX * (CDZ / 4); e += 256) {
-      const int p = e / (CDZ / 4), c0 = (e % (CDZ / 4)) * 4;
-      half4 v;
-      __builtin_memcpy(&v, dz + (((int64_t)n * H + y) * W + x0 + p) * CDZ + c0, 8);
+  for (int q = 0; q < PW; ++q)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) sdz[c0 + q][p] = v[q];
-    }
-    const int yy = wrap(y + dy, H);
-    for (int e = tid; e < WG_PIX * (CINP / 4); e += 256) {
-      const int p = e / (CINP / 4), c0 = (e % (CINP / 4)) * 4;
-      const int xx = wrap(x0 + p + dx, W);
-      half4 v;
-      __builtin_memcpy(&v, x + (((int64_t)n * H + yy) * W + xx) * CINP + c0, 8);
+    for (int t = 0; t < 9; ++t) acc[q][t] = float4v{0.f, 0.f, 0.f, 0.f};
+  float bacc = 0.f;   // bias partial of channel tid % CDZ over pixels tid / CDZ, + 256 / CDZ, ...
+  const int segs = (W + WG_SEG - 1) / WG_SEG;
+  for (int task = blockIdx.x; task < tasks; task += gridDim.x) {
+    const int n = task / (strips * segs), y0 = task / segs % strips * rows, x0 = task % segs * WG_SEG;
+    const int nrows = min(rows, H - y0), px = min(WG_SEG, W - x0);
+    const E* xi = x + (int64_t)n * H * W * CINP;
+    const E* zi = dz + (int64_t)n * H * W * CDZ;
+    half8 vz[PZ];
+    const auto load_x = [&](int y, half8 (&vx)[PX]) {
+      const E* row = xi + (int64_t)wrap(y, H) * W * CINP;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) sx[c0 + q][p] = v[q];
-    }
-    __syncthreads();
-    if (tap == 4 && tid < CDZ * 4) {
+      for (int q = 0; q < PX; ++q) {
+        const int e = min(tid + q * 256, NX - 1);
+        const int xx = (x0 + e / (CINP / 8) - 1 + W) % W;
+        vx[q] = *reinterpret_cast<const half8*>(row + (int64_t)xx * CINP + e % (CINP / 8) * 8);
+      }
+    };
+    const auto store_x = [&](int slot, const half8 (&vx)[PX]) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) bacc += (float)sdz[tid >> 2][(tid & 3) * 8 + e];
-    }
+      for (int q = 0; q < PX; ++q) {
+        const int e = tid + q * 256;
+        if (e < NX) *reinterpret_cast<half8*>(sx + (slot * SPAN + e / (CINP / 8)) * XS + e % (CINP / 8) * 8) = vx[q];
+      }
+    };
+    const auto load_z = [&](int y) {
+      const E* row = zi + ((int64_t)y * W + x0) * CDZ;
 #pragma unroll
-    for (int q = 0; q < PER_WAVE; ++q) {
-      const int t = wv * PER_WAVE + q;
-      const int mt = t / NT, nt = t % NT;
-      half8 a, b;
-      __builtin_memcpy(&a, &sdz[mt * 16 + r][g * 8], 16);
-      __builtin_memcpy(&b, &sx[nt * 16 + r][g * 8], 16);
-      acc[q] = Elem<E>::mfma(a, b, acc[q]);
+      for (int q = 0; q < PZ; ++q) {
+        const int e = min(tid + q * 256, px * (CDZ / 8) - 1);
+        vz[q] = *reinterpret_cast<const half8*>(row + e * 8);
+      }
+    };
+    const auto store_z = [&](int slot) {
+#pragma unroll
+      for (int q = 0; q < PZ; ++q) {
+        const int e = tid + q * 256;
+        if (e < NZ && e / (CDZ / 8) < px)
+          *reinterpret_cast<half8*>(sz + (slot * WG_SEG + e / (CDZ / 8)) * ZS + e % (CDZ / 8) * 8) = vz[q];
+      }
+    };
+    half8 v0[PX], v1[PX], v2[PX];
+    load_x(y0 - 1, v0);
+    load_x(y0, v1);
+    load_x(y0 + 1, v2);
+    load_z(y0);
+    __syncthreads();   // the last strip's rows are read
+    store_x(0, v0);
+    store_x(1, v1);
+    store_x(2, v2);
+    store_z(0);
+    for (int j = 0; j < nrows; ++j) {
+      // row y0 + j - 1 + i lies in slot i % 4; the row loaded here goes where row j - 2 was
+      if (j + 1 < nrows) {
+        load_x(y0 + j + 2, v0);
+        load_z(y0 + j + 1);
+      }
+      __syncthreads();
+      const E* zr = sz + (j & 1) * WG_SEG * ZS;
+      for (int p = 0; p < px; p += 32) {
+        half8 a[PW];
+#pragma unroll
+        for (int q = 0; q < PW; ++q) a[q] = read_tr(zr + p * ZS + (mt0 + q) * 16, ZS);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          const half8 b = read_tr(sx + ((j + t / 3 & 3) * SPAN + p + t % 3) * XS + nt * 16, XS);
+#pragma unroll
+          for (int q = 0; q < PW; ++q) acc[q][t] = Elem<E>::mfma(a[q], b, acc[q][t]);
+        }
+      }
+      for (int p = tid / CDZ; p < px; p += 256 / CDZ) bacc += (float)zr[p * ZS + tid % CDZ];
+      if (j + 1 < nrows) {
+        store_x(j + 3 & 3, v0);
+        store_z(j + 1 & 1);
+      }
     }
   }
   // partial[bx][tap][co][ci]
-  float* dst = partial + ((int64_t)blockIdx.x * 9 + tap) * CDZ * CINP;
+  float* dst = partial + (int64_t)blockIdx.x * 9 * CDZ * CINP;
 #pragma unroll
-  for (int q = 0; q < PER_WAVE; ++q) {
-    const int t = wv * PER_WAVE + q;
-    const int mt = t / NT, nt = t % NT;
+  for (int q = 0; q < PW; ++q)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) dst[(mt * 16 + g * 4 + e) * CINP + nt * 16 + r] = acc[q][e];
-  }
-  if (tap == 4) {
-    // the 4 lanes of one channel are consecutive lanes of one wave
-    bacc += __shfl_xor(bacc, 1);
-    bacc += __shfl_xor(bacc, 2);
-    if (tid < CDZ * 4 && (tid & 3) == 0) partial_b[(int64_t)blockIdx.x * CDZ + (tid >> 2)] = bacc;
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        dst[(t * CDZ + (mt0 + q) * 16 + g * 4 + e) * CINP + nt * 16 + r] = acc[q][t][e];
+  __syncthreads();
+  float* sb = reinterpret_cast<float*>(sx);
+  sb[tid] = bacc;
+  __syncthreads();
+  if (tid < CDZ) {
+    float b = sb[tid];
+    for (int q = 1; q < 256 / CDZ; ++q) b += sb[q * CDZ + tid];
+    partial_b[(int64_t)blockIdx.x * CDZ + tid] = b;
   }
 }
 
-// out[i] = sum over nblk rows of partial[b * len + i]: four interleaved running sums
-// (rows b = 4 j + q) added in a fixed order, so the result is deterministic
+// out[i] = sum over nblk rows of partial[b * len + i], and behind them the bias
+// gradients: a workgroup sums 64 columns, wave q the rows b = 4 j + q in eight running
+// sums, all added in a fixed order, so the result is deterministic
 __global__ void __launch_bounds__(256) sum_partials_kernel(const float* __restrict__ partial, int nblk, int len,
-                                                           float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
-  float s[4] = {0.f, 0.f, 0.f, 0.f};
-  int b = 0;
-  for (; b + 4 <= nblk; b += 4) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) s[q] += partial[(int64_t)(b + q) * len + i];
+                                                           float* __restrict__ out,
+                                                           const float* __restrict__ partial_b, int len_b,
+                                                           float* __restrict__ out_b) {
+  __shared__ float sh[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int i = blockIdx.x * 64 + lane, n = len;
+  const float* src = partial;
+  float* dst = out;
+  if (blockIdx.x * 64 >= len) {   // len is a multiple of 64
+    i -= len;
+    n = len_b;
+    src = partial_b;
+    dst = out_b;
   }
-  for (; b < nblk; ++b) s[0] += partial[(int64_t)b * len + i];
-  out[i] = (s[0] + s[1]) + (s[2] + s[3]);
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (i < n) {
+    int b = wv;
+    for (; b + 28 < nblk; b += 32) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s[q] += src[(int64_t)(b + 4 * q) * n + i];
+    }
+    for (; b < nblk; b += 4) s[0] += src[(int64_t)b * n + i];
+  }
+  sh[wv][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  __syncthreads();
+  if (wv == 0 && i < n) dst[i] = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
 }
 
 // Masked mean-square loss over the 48 value channels of 64; dY = 2 gscale (y - t) as E
@@ -666,6 +793,36 @@ __global__ void __launch_bounds__(256) adam_kernel(float* __restrict__ w, float*
   m[i] = mi;
   v[i] = vi;
   *param -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+}
+
+// One Adam step on every layer of a network and its 16-bit operands from the new
+// weights, in one launch: the thread of weight (tap, ci, co) writes its places of the
+// forward and backward operands itself (the arithmetic of adam_kernel and pack_kernel)
+struct NetLayers {
+  lbm_sur_layer l[LBM_SUR_MAX_LAYERS];
+};
+
+template <typename E>
+__global__ void __launch_bounds__(256) adam_net_kernel(NetLayers net, float lr, float b1, float b2, float eps,
+                                                       float c1, float c2) {
+  const lbm_sur_layer& l = net.l[blockIdx.y];
+  const int cin = l.cin, cout = l.cout, nw = 9 * cin * cout;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nw + cout) return;
+  const int tap = i / (cin * cout), ci = (i / cout) % cin, co = i % cout;
+  const bool weight = i < nw;
+  const float grad = weight ? l.dwt[((int64_t)tap * cout + co) * cin + ci] : l.db[i - nw];
+  float* param = weight ? l.w + i : l.b + (i - nw);
+  const float mi = b1 * l.m[i] + (1.f - b1) * grad;
+  const float vi = b2 * l.v[i] + (1.f - b2) * grad * grad;
+  l.m[i] = mi;
+  l.v[i] = vi;
+  const float p = *param - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  *param = p;
+  if (weight) {
+    ((E*)l.afwd)[((int64_t)co * 9 + tap) * cin + ci] = (E)p;
+    if (l.abwd) ((E*)l.abwd)[((int64_t)ci * 9 + 8 - tap) * cout + co] = (E)p;
+  }
 }
 
 // ------------------------------------------------------- state <-> network
@@ -926,17 +1083,24 @@ int with_elem(int elem, const char* what, F&& f) {
 template <typename E, int CINP, int COUTP, int EPI>
 int conv_launch(const void* in, const void* wpk, const float* bias, const void* zin, void* out, void* zout, int N,
                 int H, int W, const ApplyArgs& ap, hipStream_t s) {
-  constexpr size_t lds = ((size_t)COUTP * (9 * CINP + 8) + 3 * 66 * (CINP + 8)) * EB;
+  constexpr size_t lds = conv_lds<CINP, COUTP>();
   static_assert(lds <= 160 * 1024, "LDS budget");
-  static bool attr = false;  // allow more than 64 KiB of dynamic LDS once per instantiation
-  if (!attr) {
-    LBM_CHECK_HIP(hipFuncSetAttribute((const void*)conv3x3_kernel<E, CINP, COUTP, EPI>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = true;
+  if constexpr (lds > 64 * 1024) {
+    static bool attr = false;  // allow more than 64 KiB of dynamic LDS once per instantiation
+    if (!attr) {
+      LBM_CHECK_HIP(hipFuncSetAttribute((const void*)conv3x3_kernel<E, CINP, COUTP, EPI>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      attr = true;
+    }
   }
-  const int64_t groups = (int64_t)N * H * ((W + 63) / 64);
+  // strips of up to CONV_ROWS rows, shorter where that leaves fewer than CONV_GROUPS workgroups
+  const int segs = (W + CONV_SEG - 1) / CONV_SEG;
+  int rows = (int)((int64_t)N * segs * H / CONV_GROUPS);
+  rows = rows < 1 ? 1 : (rows > CONV_ROWS ? CONV_ROWS : rows);
+  const int strips = (H + rows - 1) / rows;
+  const int64_t groups = (int64_t)N * strips * segs;
   conv3x3_kernel<E, CINP, COUTP, EPI><<<(unsigned)groups, 256, lds, s>>>(
-      (const E*)in, (const E*)wpk, bias, (const E*)zin, out, (E*)zout, N, H, W, ap);
+      (const E*)in, (const E*)wpk, bias, (const E*)zin, out, (E*)zout, H, W, rows, strips, ap);
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1069,32 +1233,37 @@ int lbm_sur_wgrad(const void* d_x, int cinp, const void* d_dz, int cdz, int N, i
   LBM_REQUIRE(N > 0 && H > 0 && W > 0 && W % WG_PIX == 0, "wgrad: W must be a positive multiple of %d (got %d)",
               WG_PIX, W);
   LBM_REQUIRE((int64_t)N * H * W * 64 < ((int64_t)1 << 31), "wgrad: too many pixels");
-  const int nblk = SUR_WGRAD_BLOCKS;
   const int64_t len = 9 * (int64_t)cdz * cinp;
+  // strips of rows, as many as there are workgroups where the images allow it
+  const int segs = (W + WG_SEG - 1) / WG_SEG;
+  int strips = SUR_WGRAD_BLOCKS / (N * segs);
+  strips = strips < 1 ? 1 : (strips > H ? H : strips);
+  const int rows = (H + strips - 1) / strips;
+  strips = (H + rows - 1) / rows;
+  const int tasks = N * strips * segs;
+  const int nblk = tasks < SUR_WGRAD_BLOCKS ? tasks : SUR_WGRAD_BLOCKS;
   float* pb = d_partial + (int64_t)nblk * len;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(nblk, 9);
   const int rc = with_elem(elem, "wgrad", [&](auto tag) -> int {
     using E = typename decltype(tag)::type;
     const E* x = (const E*)d_x;
     const E* dz = (const E*)d_dz;
-    if (cinp == 64 && cdz == 64)
-      conv3x3_wgrad_kernel<E, 64, 64><<<grid, 256, 0, s>>>(x, dz, d_partial, pb, N, H, W);
-    else if (cinp == 64 && cdz == 32)
-      conv3x3_wgrad_kernel<E, 64, 32><<<grid, 256, 0, s>>>(x, dz, d_partial, pb, N, H, W);
-    else if (cinp == 32 && cdz == 32)
-      conv3x3_wgrad_kernel<E, 32, 32><<<grid, 256, 0, s>>>(x, dz, d_partial, pb, N, H, W);
-    else if (cinp == 32 && cdz == 64)
-      conv3x3_wgrad_kernel<E, 32, 64><<<grid, 256, 0, s>>>(x, dz, d_partial, pb, N, H, W);
-    else
-      LBM_REQUIRE(false, "wgrad: unsupported shape cinp=%d cdz=%d", cinp, cdz);
-    return 0;
+#define SUR_WGRAD(CI, CZ)                                                                                    \
+  if (cinp == CI && cdz == CZ) {                                                                             \
+    conv3x3_wgrad_kernel<E, CI, CZ><<<nblk, 256, 0, s>>>(x, dz, d_partial, pb, H, W, rows, strips, tasks); \
+    return 0;                                                                                                \
+  }
+    SUR_WGRAD(64, 64)
+    SUR_WGRAD(64, 32)
+    SUR_WGRAD(32, 32)
+    SUR_WGRAD(32, 64)
+#undef SUR_WGRAD
+    LBM_REQUIRE(false, "wgrad: unsupported shape cinp=%d cdz=%d", cinp, cdz);
   });
   if (rc) return rc;
   LBM_CHECK_HIP(hipGetLastError());
-  sum_partials_kernel<<<blocks_for(len), 256, 0, s>>>(d_partial, nblk, (int)len, d_dwt);
-  LBM_CHECK_HIP(hipGetLastError());
-  sum_partials_kernel<<<1, 256, 0, s>>>(pb, nblk, cdz, d_db);
+  sum_partials_kernel<<<(unsigned)(len / 64 + (cdz + 63) / 64), 256, 0, s>>>(d_partial, nblk, (int)len, d_dwt, pb, cdz,
+                                                                           d_db);
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1142,6 +1311,33 @@ int lbm_sur_adam(float* d_w, float* d_b, float* d_m, float* d_v, const float* d_
   const int n = 9 * cin * cout + cout;
   adam_kernel<<<blocks_for(n), 256, 0, (hipStream_t)stream>>>(d_w, d_b, d_m, d_v, d_dwt, d_db, cin, cout, cinp,
                                                               coutp, lr, b1, b2, eps, c1, c2);
+  LBM_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+
+int lbm_sur_adam_net(const lbm_sur_layer* layers, int nlayers, float lr, float b1, float b2, float eps, int step,
+                     int elem, void* stream) {
+  LBM_REQUIRE(layers != nullptr && nlayers >= 1 && nlayers <= LBM_SUR_MAX_LAYERS, "adam_net: 1 to %d layers",
+              LBM_SUR_MAX_LAYERS);
+  LBM_REQUIRE(step >= 1, "adam_net: step must be >= 1");
+  NetLayers net{};
+  int most = 0;
+  for (int i = 0; i < nlayers; ++i) {
+    const lbm_sur_layer& l = layers[i];
+    LBM_REQUIRE(l.cin > 0 && l.cout > 0 && l.cin <= 64 && l.cout <= 64, "adam_net: channel counts out of range");
+    LBM_REQUIRE(l.w && l.b && l.m && l.v && l.dwt && l.db && l.afwd, "adam_net: NULL buffer");
+    net.l[i] = l;
+    const int n = 9 * l.cin * l.cout + l.cout;
+    most = n > most ? n : most;
+  }
+  const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
+  const int rc = with_elem(elem, "adam_net", [&](auto tag) -> int {
+    using E = typename decltype(tag)::type;
+    adam_net_kernel<E><<<dim3(blocks_for(most), (unsigned)nlayers), 256, 0, (hipStream_t)stream>>>(net, lr, b1, b2, eps,
+                                                                                                 c1, c2);
+    return 0;
+  });
+  if (rc) return rc;
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }

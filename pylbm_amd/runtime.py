@@ -117,6 +117,12 @@ class LbmSurNet(ctypes.Structure):
                 ("bias", ctypes.c_void_p * 4), ("hidden", ctypes.c_int32), ("elem", ctypes.c_int32)]
 
 
+class LbmSurLayer(ctypes.Structure):
+    _fields_ = [("w", ctypes.c_void_p), ("b", ctypes.c_void_p), ("m", ctypes.c_void_p), ("v", ctypes.c_void_p),
+                ("dwt", ctypes.c_void_p), ("db", ctypes.c_void_p), ("afwd", ctypes.c_void_p),
+                ("abwd", ctypes.c_void_p), ("cin", ctypes.c_int32), ("cout", ctypes.c_int32)]
+
+
 SURROGATE_SIGNATURES = {
     "lbm_sur_run": ([ctypes.POINTER(LbmSurNet), _P, _P, _FP, _FP, _FP, _I64, _I, _I, _I, _P], _I),
     "lbm_sur_conv": ([_P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P], _I),
@@ -126,6 +132,7 @@ SURROGATE_SIGNATURES = {
     "lbm_sur_mse": ([_P, _P, _I64, _F, _P, _P, ctypes.POINTER(_D), _I, _P], _I),
     "lbm_sur_pack": ([_P, _I, _I, _I, _I, _P, _P, _I, _P], _I),
     "lbm_sur_adam": ([_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _F, _F, _F, _I, _P], _I),
+    "lbm_sur_adam_net": ([ctypes.POINTER(LbmSurLayer), _I, _F, _F, _F, _F, _I, _I, _P], _I),
     "lbm_sur_make_input": ([_P, _I, _I, _I, _FP, _FP, _P, _I, _P], _I),
     "lbm_sur_make_target": ([_P, _P, _I, _I, _I, _FP, _P, _P], _I),
     "lbm_sur_moments_to_state": ([_P, ctypes.POINTER(LbmLayout), _I, _I, _I, _I, _I, _P, _P], _I),

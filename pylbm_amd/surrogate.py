@@ -245,16 +245,14 @@ class SurrogateNet:
                 grad_in = out
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, eps_scale=1.0):
-        """One Adam step on every layer, then repack the 16-bit operands."""
+        """One Adam step on every layer and their 16-bit operands repacked, in one launch."""
         self.step += 1
         ch = self.ch
-        for i in range(4):
-            self.rt.check(self.lib.lbm_sur_adam(ctypes.c_void_p(self.w[i]), ctypes.c_void_p(self.b[i]),
-                                                ctypes.c_void_p(self.m[i]), ctypes.c_void_p(self.v[i]),
-                                                ctypes.c_void_p(self.dwt[i]), ctypes.c_void_p(self.db[i]),
-                                                ch[i], ch[i + 1], ch[i], ch[i + 1], float(lr), float(b1), float(b2),
-                                                float(eps * eps_scale), self.step, self.stream), "lbm_sur_adam")
-        self.pack()
+        layers = (rtm.LbmSurLayer * 4)(*[
+            rtm.LbmSurLayer(self.w[i], self.b[i], self.m[i], self.v[i], self.dwt[i], self.db[i], self.afwd[i],
+                            self.abwd[i], ch[i], ch[i + 1]) for i in range(4)])
+        self.rt.check(self.lib.lbm_sur_adam_net(layers, 4, float(lr), float(b1), float(b2), float(eps * eps_scale),
+                                                self.step, self.elem, self.stream), "lbm_sur_adam_net")
 
     def train_step(self, n, lr, sync=False):
         """forward, loss-scaled MSE gradient, backward, Adam (same step as the unscaled loss)."""
