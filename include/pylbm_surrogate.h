@@ -92,7 +92,7 @@ typedef struct lbm_sur_net {
 int lbm_sur_run(lbm_sur_net* net, const float* d_src, float* d_state, const float* dscale, const float* shift,
                 const float* scale, int64_t nsteps, int N, int H, int W, void* stream);
 
-/* number of partial sums lbm_sur_wgrad uses, at most */
+/* number of partial sums lbm_sur_wgrad uses */
 int lbm_sur_wgrad_blocks(void);
 
 /*

@@ -15,8 +15,8 @@
 //     v_mfma_f32_16x16x32_f16 / _bf16, 32 input channels of one tap per K step.  A wave
 //     computes 16 consecutive pixels of one row for MT * 16 output channels.
 //   weight gradient: dW[tap]^T[co][ci] = sum_p dZ[p][co] X[p + d_tap][ci], K = pixels,
-//     operands staged transposed in LDS (aligned 16-byte reads), one tap per
-//     workgroup row of the grid, per-workgroup partials reduced in a second pass
+//     operands staged in LDS as they lie in memory and read transposed, the three taps
+//     of a row offset per workgroup, per-workgroup partials reduced in a second pass
 //     in a fixed order (deterministic).
 // Lane layouts (checked on the device against a CPU product; the same for both
 // element types): for 16x16x32, lane l
@@ -59,8 +59,7 @@ constexpr int EPI_BWD = 2;    // g = acc * silu'(z_in): store E
 constexpr int EPI_APPLY = 3;  // fine state += (acc + b) * dscale, next network input
 
 constexpr int WG_PIX = 32;             // pixels of one weight-gradient K step
-constexpr int WG_SEG = 64;             // pixels of a weight-gradient row segment
-constexpr int SUR_WGRAD_BLOCKS = 256;  // weight-gradient workgroups, at most: one per CU
+constexpr int SUR_WGRAD_BLOCKS = 64;   // partial sums of a weight gradient
 
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
 
@@ -547,15 +546,16 @@ __global__ void __launch_bounds__(64 * FUSED_WAVES) fused_step_kernel(const E* _
 // Weight and bias gradients: dW[tap]^T[co][ci] = sum over pixels p of dZ[p][co] X[p + d_tap][ci].
 // The pixels are the K dimension of the MFMA, so both operands are wanted with eight
 // pixels of one channel per lane while memory has the channels of one pixel together:
-// rows are staged in LDS as they lie in memory and read with ds_read_b64_tr_b16, which
+// pixels are staged in LDS as they lie in memory and read with ds_read_b64_tr_b16, which
 // hands lane i of 16 the values of channel i of four pixels.  A tap is then only another
-// first pixel, so one workgroup computes all nine taps from one read of dZ and X: it
-// walks down a strip of rows, 64 pixels wide, with the next row's loads in flight while
-// the MFMAs of this row run (X: a ring of four rows, dZ: two).  A wave keeps one input
-// tile of 16 channels and MT * NT / 4 output tiles, 9 accumulators each.
-// Bound by latency and the partial sums (8 x 128 x 128 pixels: the bytes take 4-6 us, the
-// MFMAs 1-2).  32 x 32 channels 13 us, 64 x 32 17 us, 32 x 64 19 us; one workgroup row
-// per tap, operands transposed on their way into LDS 16 bits at a time, took 48, 90 and 83.
+// first pixel, so a workgroup computes the three taps of one row offset for 32 x 32
+// channels from one read of dZ and X.  Its pixels are the blocks of 32 with index
+// bx mod 64, summed one after the other: the sums have a fixed order that depends on
+// neither the taps, the channels nor the GPU, and a bias gradient that cancels to a
+// thousandth of its terms (a zero-mean loss gradient) keeps its value from release to
+// release.  64 x 3 x (1, 2 or 4 channel quarters) workgroups; groups of the same pixels
+// lie 64 apart in the grid, on one XCD and its L2.  Two stages of four blocks are in
+// flight in registers behind the one in LDS.
 template <typename E>
 __device__ __forceinline__ typename Elem<E>::v8 read_tr(const E* base, int stride) {
   // lane (g, i): pixels 8 g + [0, 8), channel i of the 16 at base (stride elements per pixel)
@@ -574,123 +574,115 @@ __device__ __forceinline__ typename Elem<E>::v8 read_tr(const E* base, int strid
 template <typename E, int CINP, int CDZ>
 __global__ void __launch_bounds__(256) conv3x3_wgrad_kernel(const E* __restrict__ x, const E* __restrict__ dz,
                                                             float* __restrict__ partial,
-                                                            float* __restrict__ partial_b, int H, int W, int rows,
-                                                            int strips, int tasks) {
+                                                            float* __restrict__ partial_b, int N, int H, int W) {
   typedef typename Elem<E>::v8 half8;
-  constexpr int NT = CINP / 16, PW = CDZ / 16 * NT / 4;   // output tiles per wave
-  constexpr int SPAN = WG_SEG + 2, XS = CINP + 8, ZS = CDZ + 8;   // padded pixels: 16 B apart in the banks
-  constexpr int NX = SPAN * (CINP / 8), NZ = WG_SEG * (CDZ / 8);   // 16-byte items of a row
-  constexpr int PX = (NX + 255) / 256, PZ = (NZ + 255) / 256;
-  __shared__ __attribute__((aligned(16))) E sx[4 * SPAN * XS];
-  __shared__ __attribute__((aligned(16))) E sz[2 * WG_SEG * ZS];
+  constexpr int U = 4, SPAN = WG_PIX + 2, CS = 32 + 8;   // a block per wave; padded pixels: 16 B apart in the banks
+  constexpr int NX = SPAN * 4, PX = (NX + 63) / 64, PZ = WG_PIX * 4 / 64;   // 16-byte items of a block
+  __shared__ __attribute__((aligned(16))) E sx[2][U * SPAN * CS];
+  __shared__ __attribute__((aligned(16))) E sz[2][U * WG_PIX * CS];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = lane >> 4, r = lane & 15;
-  const int nt = wv % NT, mt0 = wv / NT * PW;
-  float4v acc[PW][9];
+  const int bx = blockIdx.x, dy = (int)blockIdx.y - 1;
+  const int ci0 = (int)blockIdx.z % (CINP / 32) * 32, co0 = (int)blockIdx.z / (CINP / 32) * 32;
+  const int nt = wv & 1, mt = wv >> 1;
+  const bool bias = dy == 0 && ci0 == 0 && tid < 128;
+  float4v acc[3];
 #pragma unroll
-  for (int q = 0; q < PW; ++q)
-#pragma unroll
-    for (int t = 0; t < 9; ++t) acc[q][t] = float4v{0.f, 0.f, 0.f, 0.f};
-  float bacc = 0.f;   // bias partial of channel tid % CDZ over pixels tid / CDZ, + 256 / CDZ, ...
-  const int segs = (W + WG_SEG - 1) / WG_SEG;
-  for (int task = blockIdx.x; task < tasks; task += gridDim.x) {
-    const int n = task / (strips * segs), y0 = task / segs % strips * rows, x0 = task % segs * WG_SEG;
-    const int nrows = min(rows, H - y0), px = min(WG_SEG, W - x0);
-    const E* xi = x + (int64_t)n * H * W * CINP;
-    const E* zi = dz + (int64_t)n * H * W * CDZ;
-    half8 vz[PZ];
-    const auto load_x = [&](int y, half8 (&vx)[PX]) {
-      const E* row = xi + (int64_t)wrap(y, H) * W * CINP;
+  for (int t = 0; t < 3; ++t) acc[t] = float4v{0.f, 0.f, 0.f, 0.f};
+  float bacc = 0.f;   // bias partial of channel tid / 4 over pixels (tid % 4) * 8 + [0, 8)
+  const int segs = W / WG_PIX, rows = N * H;
+  const int nblocks = rows * segs;
+  const int mine = bx < nblocks ? (nblocks - 1 - bx) / SUR_WGRAD_BLOCKS + 1 : 0;   // blocks bx, bx + 64, ...
+  const int stages = (mine + U - 1) / U;
+  // wave u loads the blocks u, u + 4, ... of them: the next one's row (over all images),
+  // row of its image and segment, and the step from one to the next
+  const int u0 = __builtin_amdgcn_readfirstlane(wv);
+  const int step_row = U * SUR_WGRAD_BLOCKS / segs, step_seg = U * SUR_WGRAD_BLOCKS % segs, step_y = step_row % H;
+  int next = u0;
+  int row = (bx + u0 * SUR_WGRAD_BLOCKS) / segs, seg = (bx + u0 * SUR_WGRAD_BLOCKS) % segs, y = row % H;
+  struct Stage {
+    half8 x[PX], z[PZ];
+  };
+  const auto load = [&](Stage& v) {
+    if (next < mine) {
+      const E* const xr = x + (int64_t)(row - y + wrap(y + dy, H)) * W * CINP + ci0;
+      const E* const zr = dz + ((int64_t)row * W + seg * WG_PIX) * CDZ + co0;
 #pragma unroll
       for (int q = 0; q < PX; ++q) {
-        const int e = min(tid + q * 256, NX - 1);
-        const int xx = (x0 + e / (CINP / 8) - 1 + W) % W;
-        vx[q] = *reinterpret_cast<const half8*>(row + (int64_t)xx * CINP + e % (CINP / 8) * 8);
+        const int e = min(lane + q * 64, NX - 1);
+        v.x[q] = *reinterpret_cast<const half8*>(xr + (int64_t)wrap(seg * WG_PIX + e / 4 - 1, W) * CINP + e % 4 * 8);
       }
-    };
-    const auto store_x = [&](int slot, const half8 (&vx)[PX]) {
-#pragma unroll
-      for (int q = 0; q < PX; ++q) {
-        const int e = tid + q * 256;
-        if (e < NX) *reinterpret_cast<half8*>(sx + (slot * SPAN + e / (CINP / 8)) * XS + e % (CINP / 8) * 8) = vx[q];
-      }
-    };
-    const auto load_z = [&](int y) {
-      const E* row = zi + ((int64_t)y * W + x0) * CDZ;
 #pragma unroll
       for (int q = 0; q < PZ; ++q) {
-        const int e = min(tid + q * 256, px * (CDZ / 8) - 1);
-        vz[q] = *reinterpret_cast<const half8*>(row + e * 8);
-      }
-    };
-    const auto store_z = [&](int slot) {
-#pragma unroll
-      for (int q = 0; q < PZ; ++q) {
-        const int e = tid + q * 256;
-        if (e < NZ && e / (CDZ / 8) < px)
-          *reinterpret_cast<half8*>(sz + (slot * WG_SEG + e / (CDZ / 8)) * ZS + e % (CDZ / 8) * 8) = vz[q];
-      }
-    };
-    half8 v0[PX], v1[PX], v2[PX];
-    load_x(y0 - 1, v0);
-    load_x(y0, v1);
-    load_x(y0 + 1, v2);
-    load_z(y0);
-    __syncthreads();   // the last strip's rows are read
-    store_x(0, v0);
-    store_x(1, v1);
-    store_x(2, v2);
-    store_z(0);
-    for (int j = 0; j < nrows; ++j) {
-      // row y0 + j - 1 + i lies in slot i % 4; the row loaded here goes where row j - 2 was
-      if (j + 1 < nrows) {
-        load_x(y0 + j + 2, v0);
-        load_z(y0 + j + 1);
-      }
-      __syncthreads();
-      const E* zr = sz + (j & 1) * WG_SEG * ZS;
-      for (int p = 0; p < px; p += 32) {
-        half8 a[PW];
-#pragma unroll
-        for (int q = 0; q < PW; ++q) a[q] = read_tr(zr + p * ZS + (mt0 + q) * 16, ZS);
-#pragma unroll
-        for (int t = 0; t < 9; ++t) {
-          const half8 b = read_tr(sx + ((j + t / 3 & 3) * SPAN + p + t % 3) * XS + nt * 16, XS);
-#pragma unroll
-          for (int q = 0; q < PW; ++q) acc[q][t] = Elem<E>::mfma(a[q], b, acc[q][t]);
-        }
-      }
-      for (int p = tid / CDZ; p < px; p += 256 / CDZ) bacc += (float)zr[p * ZS + tid % CDZ];
-      if (j + 1 < nrows) {
-        store_x(j + 3 & 3, v0);
-        store_z(j + 1 & 1);
+        const int e = lane + q * 64;
+        v.z[q] = *reinterpret_cast<const half8*>(zr + e / 4 * CDZ + e % 4 * 8);
       }
     }
+    next += U;
+    seg += step_seg;
+    const int c = seg >= segs ? 1 : 0;
+    seg -= c ? segs : 0;
+    row += step_row + c;
+    y += step_y + c;
+    y -= y >= H ? H : 0;
+  };
+  // one stage: store it, load the stage after the next in its place, sum it
+  const auto stage = [&](int st, Stage& v) {
+    E* const sxs = sx[st & 1];
+    E* const szs = sz[st & 1];
+#pragma unroll
+    for (int q = 0; q < PX; ++q) {
+      const int e = lane + q * 64;
+      if (e < NX) *reinterpret_cast<half8*>(sxs + (u0 * SPAN + e / 4) * CS + e % 4 * 8) = v.x[q];
+    }
+#pragma unroll
+    for (int q = 0; q < PZ; ++q) {
+      const int e = lane + q * 64;
+      *reinterpret_cast<half8*>(szs + (u0 * WG_PIX + e / 4) * CS + e % 4 * 8) = v.z[q];
+    }
+    __syncthreads();   // one per stage: the next store goes to the other buffer
+    load(v);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (st * U + u >= mine) break;
+      const half8 a = read_tr(szs + u * WG_PIX * CS + mt * 16, CS);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const half8 b = read_tr(sxs + (u * SPAN + t) * CS + nt * 16, CS);
+        acc[t] = Elem<E>::mfma(a, b, acc[t]);
+      }
+      if (bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bacc += (float)szs[(u * WG_PIX + (tid & 3) * 8 + e) * CS + (tid >> 2)];
+      }
+    }
+  };
+  Stage v0{}, v1{};
+  load(v0);
+  load(v1);
+  for (int st = 0; st < stages; st += 2) {
+    stage(st, v0);
+    if (st + 1 < stages) stage(st + 1, v1);
   }
   // partial[bx][tap][co][ci]
-  float* dst = partial + (int64_t)blockIdx.x * 9 * CDZ * CINP;
+  float* dst = partial + ((int64_t)bx * 9 + blockIdx.y * 3) * CDZ * CINP;
 #pragma unroll
-  for (int q = 0; q < PW; ++q)
+  for (int t = 0; t < 3; ++t)
 #pragma unroll
-    for (int t = 0; t < 9; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        dst[(t * CDZ + (mt0 + q) * 16 + g * 4 + e) * CINP + nt * 16 + r] = acc[q][t][e];
-  __syncthreads();
-  float* sb = reinterpret_cast<float*>(sx);
-  sb[tid] = bacc;
-  __syncthreads();
-  if (tid < CDZ) {
-    float b = sb[tid];
-    for (int q = 1; q < 256 / CDZ; ++q) b += sb[q * CDZ + tid];
-    partial_b[(int64_t)blockIdx.x * CDZ + tid] = b;
+    for (int e = 0; e < 4; ++e)
+      dst[(t * CDZ + co0 + mt * 16 + g * 4 + e) * CINP + ci0 + nt * 16 + r] = acc[t][e];
+  if (dy == 0 && ci0 == 0) {
+    // the 4 lanes of one channel are consecutive lanes of one wave
+    bacc += __shfl_xor(bacc, 1);
+    bacc += __shfl_xor(bacc, 2);
+    if (bias && (tid & 3) == 0) partial_b[(int64_t)bx * CDZ + co0 + (tid >> 2)] = bacc;
   }
 }
 
-// out[i] = sum over nblk rows of partial[b * len + i], and behind them the bias
-// gradients: a workgroup sums 64 columns, wave q the rows b = 4 j + q in eight running
-// sums, all added in a fixed order, so the result is deterministic
-__global__ void __launch_bounds__(256) sum_partials_kernel(const float* __restrict__ partial, int nblk, int len,
+// out[i] = sum over the SUR_WGRAD_BLOCKS rows of partial[b * len + i], and behind them the
+// bias gradients: a workgroup sums 64 columns, wave q the rows b = 4 j + q in order, the
+// four sums added in a fixed order, so the result is deterministic
+__global__ void __launch_bounds__(256) sum_partials_kernel(const float* __restrict__ partial, int len,
                                                            float* __restrict__ out,
                                                            const float* __restrict__ partial_b, int len_b,
                                                            float* __restrict__ out_b) {
@@ -705,16 +697,12 @@ __global__ void __launch_bounds__(256) sum_partials_kernel(const float* __restri
     src = partial_b;
     dst = out_b;
   }
-  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  float s = 0.f;
   if (i < n) {
-    int b = wv;
-    for (; b + 28 < nblk; b += 32) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) s[q] += src[(int64_t)(b + 4 * q) * n + i];
-    }
-    for (; b < nblk; b += 4) s[0] += src[(int64_t)b * n + i];
+    for (int b = 0; b < SUR_WGRAD_BLOCKS; b += 4) s += src[(int64_t)(b + wv) * n + i];
   }
-  sh[wv][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  sh[wv][lane] = s;
   __syncthreads();
   if (wv == 0 && i < n) dst[i] = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
 }
@@ -1234,24 +1222,17 @@ int lbm_sur_wgrad(const void* d_x, int cinp, const void* d_dz, int cdz, int N, i
               WG_PIX, W);
   LBM_REQUIRE((int64_t)N * H * W * 64 < ((int64_t)1 << 31), "wgrad: too many pixels");
   const int64_t len = 9 * (int64_t)cdz * cinp;
-  // strips of rows, as many as there are workgroups where the images allow it
-  const int segs = (W + WG_SEG - 1) / WG_SEG;
-  int strips = SUR_WGRAD_BLOCKS / (N * segs);
-  strips = strips < 1 ? 1 : (strips > H ? H : strips);
-  const int rows = (H + strips - 1) / strips;
-  strips = (H + rows - 1) / rows;
-  const int tasks = N * strips * segs;
-  const int nblk = tasks < SUR_WGRAD_BLOCKS ? tasks : SUR_WGRAD_BLOCKS;
-  float* pb = d_partial + (int64_t)nblk * len;
+  float* pb = d_partial + SUR_WGRAD_BLOCKS * len;
   hipStream_t s = (hipStream_t)stream;
   const int rc = with_elem(elem, "wgrad", [&](auto tag) -> int {
     using E = typename decltype(tag)::type;
     const E* x = (const E*)d_x;
     const E* dz = (const E*)d_dz;
-#define SUR_WGRAD(CI, CZ)                                                                                    \
-  if (cinp == CI && cdz == CZ) {                                                                             \
-    conv3x3_wgrad_kernel<E, CI, CZ><<<nblk, 256, 0, s>>>(x, dz, d_partial, pb, H, W, rows, strips, tasks); \
-    return 0;                                                                                                \
+#define SUR_WGRAD(CI, CZ)                                                                             \
+  if (cinp == CI && cdz == CZ) {                                                                      \
+    conv3x3_wgrad_kernel<E, CI, CZ>                                                                   \
+        <<<dim3(SUR_WGRAD_BLOCKS, 3, (CI / 32) * (CZ / 32)), 256, 0, s>>>(x, dz, d_partial, pb, N, H, W); \
+    return 0;                                                                                         \
   }
     SUR_WGRAD(64, 64)
     SUR_WGRAD(64, 32)
@@ -1262,8 +1243,7 @@ int lbm_sur_wgrad(const void* d_x, int cinp, const void* d_dz, int cdz, int N, i
   });
   if (rc) return rc;
   LBM_CHECK_HIP(hipGetLastError());
-  sum_partials_kernel<<<(unsigned)(len / 64 + (cdz + 63) / 64), 256, 0, s>>>(d_partial, nblk, (int)len, d_dwt, pb, cdz,
-                                                                           d_db);
+  sum_partials_kernel<<<(unsigned)(len / 64 + (cdz + 63) / 64), 256, 0, s>>>(d_partial, (int)len, d_dwt, pb, cdz, d_db);
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
