@@ -101,6 +101,23 @@ class _Printer(C99CodePrinter):
             return "pow(%s, %s)" % (self._print(b), self._print(e))
         raise NotImplementedError("power %s not supported" % expr)
 
+    def _print_Add(self, expr, order=None):
+        """Terms without a product first: every product is then contracted into an FMA
+        with the sum so far."""
+        terms = self._as_ordered_terms(expr, order=order)
+        plain = [t for t in terms if not (t.is_Mul and t.as_coeff_Mul()[0] != -1) and not t.is_Pow]
+        rest = [t for t in terms if t not in plain]
+        out = ""
+        for t in plain + rest:
+            text = self._print(t)
+            if not out:
+                out = text
+            elif text.startswith("-"):
+                out += " - " + text[1:]
+            else:
+                out += " + " + text
+        return out
+
 
 def _ccode(expr) -> str:
     return _Printer().doprint(expr)
@@ -160,29 +177,71 @@ class _SumBuilder:
     """Emits grouped linear combinations, reusing identical partial sums."""
 
     def __init__(self, prefix):
-        self.lines = []
+        self.sums = []      # (name, [(sign, var)])
+        self.late = []      # lines that use the sums
         self.cache = {}
         self.prefix = prefix
         self.count = 0
+
+    def _name(self):
+        self.count += 1
+        return "%s%d" % (self.prefix, self.count - 1)
 
     def _group(self, terms):
         # terms: list of (sign, var) with sign +-1
         key = tuple(sorted(terms))
         if len(terms) == 1 and terms[0][0] == 1:
             return terms[0][1]
-        if key in self.cache:
-            return self.cache[key]
-        pos = [v for s, v in terms if s > 0]
-        neg = [v for s, v in terms if s < 0]
-        if pos:
-            expr = " + ".join(pos) + "".join(" - %s" % v for v in neg)
-        else:
-            expr = "-(" + " + ".join(neg) + ")"
-        name = "%s%d" % (self.prefix, self.count)
-        self.count += 1
-        self.lines.append("const C %s = %s;" % (name, expr))
-        self.cache[key] = name
-        return name
+        if key not in self.cache:
+            self.cache[key] = self._name()
+            self.sums.append((self.cache[key], list(terms)))
+        return self.cache[key]
+
+    @property
+    def lines(self):
+        """The sums with their common pairs (a + b or a - b, up to the sign of the whole)
+        taken out, the most frequent first, then the lines that use them."""
+        sums = {name: dict((v, sg) for sg, v in terms) for name, terms in self.sums}
+        order = list(sums)
+        count, tried = self.count, set()
+        while True:
+            pairs = {}
+            for name in order:
+                vs = sorted(sums[name])
+                for i, u in enumerate(vs):
+                    for v in vs[i + 1:]:
+                        pairs.setdefault((u, v, sums[name][u] * sums[name][v]), []).append(name)
+            best = max((q for q in pairs if q not in tried and len(pairs[q]) > 1),
+                       key=lambda q: (len(pairs[q]), q), default=None)
+            if best is None:
+                break
+            tried.add(best)
+            u, v, rel = best
+            new = next((n for n in pairs[best] if len(sums[n]) == 2 and sums[n][u] > 0), None)
+            if new is None:
+                new, count = "%s%d" % (self.prefix, count), count + 1
+                sums[new] = {u: 1, v: rel}
+                order.append(new)
+            for name in pairs[best]:
+                if name != new and new not in sums[name]:
+                    sg = sums[name].pop(u)
+                    del sums[name][v]
+                    sums[name][new] = sg
+        out, done = [], set()
+
+        def emit(name):
+            if name in done or name not in sums:
+                return
+            done.add(name)
+            for v in sums[name]:
+                emit(v)
+            pos = [v for v, sg in sums[name].items() if sg > 0]
+            neg = [v for v, sg in sums[name].items() if sg < 0]
+            expr = " + ".join(pos) + "".join(" - %s" % v for v in neg) if pos else "-(" + " + ".join(neg) + ")"
+            out.append("const C %s = %s;" % (name, expr))
+        for name in order:
+            emit(name)
+        return out + self.late
 
     def combo(self, coeffs):
         """coeffs: list of (Fraction, var). Returns a C expression."""
@@ -195,7 +254,7 @@ class _SumBuilder:
         if not groups:
             return "C(0.0)"
         parts = []
-        for a in sorted(groups):
+        for a in sorted(groups, key=lambda x: (x != 1, x)):   # the sum without a product first (FMA)
             g = self._group(groups[a])
             parts.append(g if a == 1 else "%s*%s" % (_lit(a), g))
         return " + ".join(parts)
@@ -232,14 +291,11 @@ def _transform(builder, mat, invars, outvars, ksym, sig, rows_are_outputs=True):
     return lines
 
 
-def _inverse_transform(builder, inv, mvars, fvars, ksym, sig, base=None, tag=""):
-    """Lines computing fvars = [base +] inv @ mvars (entries of mvars that are None
-    are zero); with parity f_k = E_k + O_k, f_ksym = E_k - O_k."""
+def _inverse_transform(builder, inv, mvars, fvars, ksym, sig, tag=""):
+    """Lines computing fvars = inv @ mvars (entries of mvars that are None are zero);
+    with parity f_k = E_k + O_k, f_ksym = E_k - O_k."""
     ns = len(inv)
     lines = []
-
-    def plus(k, expr):
-        return "%s + (%s)" % (base[k], expr) if base is not None else expr
 
     if ksym is not None and sig is not None:
         for k in range(ns):
@@ -248,18 +304,18 @@ def _inverse_transform(builder, inv, mvars, fvars, ksym, sig, base=None, tag="")
             even = [(inv[k][i], mvars[i]) for i in range(ns) if sig[i] > 0 and mvars[i] is not None]
             odd = [(inv[k][i], mvars[i]) for i in range(ns) if sig[i] < 0 and mvars[i] is not None]
             if ksym[k] == k:
-                lines.append((fvars[k], plus(k, builder.combo(even))))
+                lines.append((fvars[k], builder.combo(even)))
                 continue
             e = "E%s%d" % (tag, k)
             o = "O%s%d" % (tag, k)
-            builder.lines.append("const C %s = %s;" % (e, builder.combo(even)))
-            builder.lines.append("const C %s = %s;" % (o, builder.combo(odd)))
-            lines.append((fvars[k], plus(k, "%s + %s" % (e, o))))
-            lines.append((fvars[ksym[k]], plus(ksym[k], "%s - %s" % (e, o))))
+            builder.late.append("const C %s = %s;" % (e, builder.combo(even)))
+            builder.late.append("const C %s = %s;" % (o, builder.combo(odd)))
+            lines.append((fvars[k], "%s + %s" % (e, o)))
+            lines.append((fvars[ksym[k]], "%s - %s" % (e, o)))
     else:
         for k in range(ns):
-            lines.append((fvars[k], plus(k, builder.combo([(inv[k][i], mvars[i]) for i in range(ns)
-                                                           if mvars[i] is not None]))))
+            lines.append((fvars[k], builder.combo([(inv[k][i], mvars[i]) for i in range(ns)
+                                                   if mvars[i] is not None])))
     return lines
 
 
@@ -333,12 +389,12 @@ def _deviation_collision_lines(spec: KernelSpec):
     for sym, e in repl:
         out.append("const C %s = %s;" % (sym, _ccode(e)))
     for i, e in zip(relaxed, red):
-        target = "C(0.0)" if e == 0 else "(%s)" % _ccode(e)
+        target = _ccode(sp.sympify(e) - msyms[i])
         if names[i] is None:
-            out.append("C dm%d = omega[%d] * (%s - m%d);" % (i, i, target, i))
+            out.append("C dm%d = omega[%d] * (%s);" % (i, i, target))
             names[i] = "dm%d" % i
         else:
-            out.append("{ const C inc = omega[%d] * (%s - m%d); dm%d += inc; m%d += inc; }" % (i, target, i, i, i))
+            out.append("{ const C inc = omega[%d] * (%s); dm%d += inc; m%d += inc; }" % (i, target, i, i))
             continue
         out.append("m%d += dm%d;" % (i, i))
     sources()
@@ -550,6 +606,7 @@ fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename 
 %(gdecl)s
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
+#pragma clang fp contract(on)
 %(coords)s
 %(decode)s
 %(f2m)s
@@ -571,6 +628,7 @@ fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename 
 __global__ void __launch_bounds__(256)
 f2m_kernel(const S* __restrict__ f, lbm_layout fl, double* __restrict__ mo, lbm_layout ml,
            const StepArgs<double> a) {
+#pragma clang fp contract(on)
   using C = double;
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= fl.n[2]) return;
@@ -586,6 +644,7 @@ template <typename S>
 __global__ void __launch_bounds__(256)
 m2f_kernel(const double* __restrict__ mi, lbm_layout ml, S* __restrict__ f, lbm_layout fl,
            const StepArgs<double> a) {
+#pragma clang fp contract(on)
   using C = double;
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= fl.n[2]) return;
@@ -599,6 +658,7 @@ m2f_kernel(const double* __restrict__ mi, lbm_layout ml, S* __restrict__ f, lbm_
 
 __global__ void __launch_bounds__(256)
 equilibrium_kernel(double* __restrict__ mo, lbm_layout ml) {
+#pragma clang fp contract(on)
   using C = double;
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= ml.n[2]) return;
@@ -631,6 +691,7 @@ transport_kernel(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typ
 
 __global__ void __launch_bounds__(256)
 relaxation_kernel(double* __restrict__ mo, lbm_layout ml, const StepArgs<double> a) {
+#pragma clang fp contract(on)
   using C = double;
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= ml.n[2]) return;
@@ -646,6 +707,7 @@ relaxation_kernel(double* __restrict__ mo, lbm_layout ml, const StepArgs<double>
 
 __global__ void __launch_bounds__(256)
 source_term_kernel(double* __restrict__ mo, lbm_layout ml, const StepArgs<double> a) {
+#pragma clang fp contract(on)
   using C = double;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.nin[2]) return;
@@ -678,6 +740,7 @@ template <typename S>
 __global__ void __launch_bounds__(256)
 eq_m2f_kernel(const double* __restrict__ mo, lbm_layout ml, S* __restrict__ f, lbm_layout fl,
               const StepArgs<double> a) {
+#pragma clang fp contract(on)
   using C = double;
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= fl.n[2]) return;
@@ -1165,6 +1228,7 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
 %(tb_sub)s
 %(tb_gdecl)s
       {
+#pragma clang fp contract(on)
 %(tb_coords)s
 %(tb_decode)s
 %(tb_f2m)s
@@ -1383,9 +1447,9 @@ def generate_source(spec: KernelSpec) -> str:
         coll_dev, dm_names = _deviation_collision_lines(spec)
         bd = _SumBuilder("rd")
         m2f_dev_lines = _inverse_transform(bd, iM, dm_names, ["g%d" % k for k in range(ns)], ksym, sig_m2f,
-                                           base=fvars, tag="d")
+                                           tag="d")
         m2f_dev_block = bd.lines + ["const C %s = %s;" % (o, e) for o, e in m2f_dev_lines]
-        stores_dev = ["G%d[j] = Codec<S>::encode_dev(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
+        stores_dev = ["G%d[j] = Codec<S>::advance(L%d[j], f%d, g%d, a.wshift[%d]);" % (k, k, k, k, k) for k in range(ns)]
 
     # ---------------------------------------------------------- f2m / m2f / eq
     b3 = _SumBuilder("p")
