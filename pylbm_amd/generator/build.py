@@ -26,7 +26,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -ffp-contract=off: the compiler contracts nothing by itself, so the kernel variants that
 # share lines (halo / wrap reads, vector widths, several steps per launch, equilibrium +
 # m2f fused or not) give the same bits wherever they compute the same cell, whatever
-# the compiler's scheduling of each variant.  The blocks of generated arithmetic turn the
+# the compiler's scheduling of each variant.  Blocks of generated arithmetic may turn the
 # contraction of a product and a sum within one statement on: that one is made by the
 # front end from the text of the statement, the same in every variant, and saves a
 # quarter of the arithmetic (D3Q19 FP32 collision 396 -> 288 instructions with shared sums)

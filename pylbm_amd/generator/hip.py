@@ -101,9 +101,15 @@ class _Printer(C99CodePrinter):
             return "pow(%s, %s)" % (self._print(b), self._print(e))
         raise NotImplementedError("power %s not supported" % expr)
 
+    def __init__(self, fuse):
+        super().__init__()
+        self.fuse = fuse
+
     def _print_Add(self, expr, order=None):
-        """Terms without a product first: every product is then contracted into an FMA
-        with the sum so far."""
+        """With fuse the terms without a product come first: every product is then
+        contracted into an FMA with the sum so far."""
+        if not self.fuse:
+            return super()._print_Add(expr, order=order)
         terms = self._as_ordered_terms(expr, order=order)
         plain = [t for t in terms if not (t.is_Mul and t.as_coeff_Mul()[0] != -1) and not t.is_Pow]
         rest = [t for t in terms if t not in plain]
@@ -119,8 +125,8 @@ class _Printer(C99CodePrinter):
         return out
 
 
-def _ccode(expr) -> str:
-    return _Printer().doprint(expr)
+def _ccode(expr, fuse=True) -> str:
+    return _Printer(fuse).doprint(expr)
 
 
 # ----------------------------------------------------------------- structure
@@ -174,9 +180,11 @@ def _row_parities(mat, ksym, by_rows=True):
 
 
 class _SumBuilder:
-    """Emits grouped linear combinations, reusing identical partial sums."""
+    """Emits grouped linear combinations, reusing identical partial sums; with fuse also
+    the common pairs of different sums, and ordered for the contraction of products."""
 
-    def __init__(self, prefix):
+    def __init__(self, prefix, fuse=True):
+        self.fuse = fuse
         self.sums = []      # (name, [(sign, var)])
         self.late = []      # lines that use the sums
         self.cache = {}
@@ -204,7 +212,7 @@ class _SumBuilder:
         sums = {name: dict((v, sg) for sg, v in terms) for name, terms in self.sums}
         order = list(sums)
         count, tried = self.count, set()
-        while True:
+        while self.fuse:
             pairs = {}
             for name in order:
                 vs = sorted(sums[name])
@@ -254,7 +262,8 @@ class _SumBuilder:
         if not groups:
             return "C(0.0)"
         parts = []
-        for a in sorted(groups, key=lambda x: (x != 1, x)):   # the sum without a product first (FMA)
+        # with fuse the sum without a product first
+        for a in sorted(groups, key=lambda x: (self.fuse and x != 1, x)):
             g = self._group(groups[a])
             parts.append(g if a == 1 else "%s*%s" % (_lit(a), g))
         return " + ".join(parts)
@@ -328,14 +337,14 @@ def _deviation_eq(expr, full, rest):
     return e
 
 
-def _collision_lines(spec: KernelSpec, with_sources: bool):
+def _collision_lines(spec: KernelSpec, with_sources: bool, fuse=True):
     """Full-value collision (FP64, as pylbm): sources, relax, sources on m0..m{ns-1}."""
     ns, nc = spec.ns, spec.nconsm
     out = []
 
     def sources():
         for idx, expr in spec.sources:
-            out.append("m%d = m%d + half_dt * (%s);" % (idx, idx, _ccode(sp.sympify(expr))))
+            out.append("m%d = m%d + half_dt * (%s);" % (idx, idx, _ccode(sp.sympify(expr), fuse)))
 
     if with_sources and spec.sources:
         sources()
@@ -343,15 +352,15 @@ def _collision_lines(spec: KernelSpec, with_sources: bool):
     repl, red = sp.cse([spec.eq[i] for i in relaxed], symbols=sp.numbered_symbols("q_"),
                        optimizations="basic")
     for sym, e in repl:
-        out.append("const C %s = %s;" % (sym, _ccode(e)))
+        out.append("const C %s = %s;" % (sym, _ccode(e, fuse)))
     for i, e in zip(relaxed, red):
-        out.append("m%d = one_minus[%d] * m%d + omega[%d] * (%s);" % (i, i, i, i, _ccode(e)))
+        out.append("m%d = one_minus[%d] * m%d + omega[%d] * (%s);" % (i, i, i, i, _ccode(e, fuse)))
     if with_sources and spec.sources:
         sources()
     return out
 
 
-def _deviation_collision_lines(spec: KernelSpec):
+def _deviation_collision_lines(spec: KernelSpec, fuse):
     """Collision of the FP32-compute formats, in increments.
 
     The m_i are moments of d = f - w (w the rest populations of the reference
@@ -380,16 +389,19 @@ def _deviation_collision_lines(spec: KernelSpec):
     def sources():
         for idx, expr in spec.sources:
             e = sp.sympify(expr).xreplace(full)
-            out.append("{ const C inc = half_dt * (%s); m%d += inc; dm%d += inc; }" % (_ccode(e), idx, idx))
+            out.append("{ const C inc = half_dt * (%s); m%d += inc; dm%d += inc; }" % (_ccode(e, fuse), idx, idx))
 
     sources()
     relaxed = [i for i in range(nc, ns) if spec.s[i] != 0]
     eqs = [_deviation_eq(spec.eq[i], full, rest) for i in relaxed]
     repl, red = sp.cse(eqs, symbols=sp.numbered_symbols("q_"), optimizations="basic")
     for sym, e in repl:
-        out.append("const C %s = %s;" % (sym, _ccode(e)))
+        out.append("const C %s = %s;" % (sym, _ccode(e, fuse)))
     for i, e in zip(relaxed, red):
-        target = _ccode(sp.sympify(e) - msyms[i])
+        if fuse:
+            target = _ccode(sp.sympify(e) - msyms[i])
+        else:
+            target = "%s - m%d" % ("C(0.0)" if e == 0 else "(%s)" % _ccode(e, False), i)
         if names[i] is None:
             out.append("C dm%d = omega[%d] * (%s);" % (i, i, target))
             names[i] = "dm%d" % i
@@ -416,25 +428,25 @@ def _relative_collision_lines(spec: KernelSpec):
     msyms = spec.msyms
     out = []
     for d, e in enumerate(spec.rel_vel):
-        out.append("const C ru%d = %s;" % (d, _ccode(e)))
+        out.append("const C ru%d = %s;" % (d, _ccode(e, False)))
     Tu = [[sp.sympify(c) for c in r] for r in spec.Tu]
     Tmu = [[sp.sympify(c) for c in r] for r in spec.Tmu]
 
     def rows(mat, vec, which, prefix):
         exprs = [sum((mat[i][j] * vec[j] for j in range(ns) if mat[i][j] != 0), sp.Integer(0)) for i in which]
         repl, red = sp.cse(exprs, symbols=sp.numbered_symbols(prefix), optimizations="basic")
-        lines = ["const C %s = %s;" % (sym, _ccode(e)) for sym, e in repl]
+        lines = ["const C %s = %s;" % (sym, _ccode(e, False)) for sym, e in repl]
         return lines, red
 
     # relative moments of the pulled populations
     lines, red = rows(Tu, msyms, range(ns), "tr_")
     out += lines
-    out += ["const C mr%d = %s;" % (i, _ccode(e)) for i, e in zip(range(ns), red)]
+    out += ["const C mr%d = %s;" % (i, _ccode(e, False)) for i, e in zip(range(ns), red)]
     out += ["m%d = mr%d;" % (i, i) for i in range(nc, ns)]
 
     def sources():
         for idx, expr in spec.sources:
-            out.append("m%d = m%d + half_dt * (%s);" % (idx, idx, _ccode(sp.sympify(expr))))
+            out.append("m%d = m%d + half_dt * (%s);" % (idx, idx, _ccode(sp.sympify(expr), False)))
 
     sources()
     relaxed = [i for i in range(nc, ns) if spec.s[i] != 0]
@@ -442,12 +454,12 @@ def _relative_collision_lines(spec: KernelSpec):
     lines, red = rows(Tu, eqv, relaxed, "te_")
     out += lines
     for i, e in zip(relaxed, red):
-        out.append("m%d = one_minus[%d] * m%d + omega[%d] * (%s);" % (i, i, i, i, _ccode(e)))
+        out.append("m%d = one_minus[%d] * m%d + omega[%d] * (%s);" % (i, i, i, i, _ccode(e, False)))
     out += ["m%d = mr%d;" % (i, i) for i in range(nc)]
     sources()
     lines, red = rows(Tmu, msyms, range(ns), "ta_")
     out += lines
-    out += ["const C ma%d = %s;" % (i, _ccode(e)) for i, e in zip(range(ns), red)]
+    out += ["const C ma%d = %s;" % (i, _ccode(e, False)) for i, e in zip(range(ns), red)]
     return out, ["ma%d" % i for i in range(ns)]
 
 
@@ -606,15 +618,15 @@ fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename 
 %(gdecl)s
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
-#pragma clang fp contract(on)
 %(coords)s
 %(decode)s
-%(f2m)s
   if constexpr (DEV) {
+%(f2m_dev)s
 %(coll_dev)s
 %(m2f_dev)s
 %(stores_dev)s
   } else {
+%(f2m)s
 %(coll)s
 %(m2f)s
 %(stores)s
@@ -1228,15 +1240,15 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
 %(tb_sub)s
 %(tb_gdecl)s
       {
-#pragma clang fp contract(on)
 %(tb_coords)s
 %(tb_decode)s
-%(tb_f2m)s
       if constexpr (DEV) {
+%(tb_f2m_dev)s
 %(tb_coll_dev)s
 %(tb_m2f_dev)s
 %(tb_stores_dev)s
       } else {
+%(tb_f2m)s
 %(tb_coll)s
 %(tb_m2f)s
 %(tb_stores)s
@@ -1430,26 +1442,37 @@ def generate_source(spec: KernelSpec) -> str:
                   % (k, k, k, k, k) for k in range(ns)]
     vstores = ["vstore<S, VEC>(fn + ((I)a.dst_off[%d] + cell), G%d);" % (k, k) for k in range(ns)]
 
-    b1 = _SumBuilder("p")
-    f2m_lines = _transform(b1, M, fvars, mvars, ksym, sig_f2m)
-    f2m_block = b1.lines + ["C %s = %s;" % (o, e) for o, e in f2m_lines]
+    # The arithmetic of the step.  With fuse (FP64, and every format in 3D) moments share
+    # partial sums and products are contracted: a quarter fewer instructions.  The
+    # FP32-compute formats of 1D and 2D schemes keep the rounding of every single product
+    # and sum: their moments are read back in FP64, where another rounding would show
+    # (6e-8) as a change of results.
+    fuse, fuse_dev = not rel, not rel and dim == 3
+
+    def f2m_of(on):
+        b1 = _SumBuilder("p", on)
+        f2m_lines = _transform(b1, M, fvars, mvars, ksym, sig_f2m)
+        return ((["#pragma clang fp contract(on)"] if on else [])
+                + b1.lines + ["C %s = %s;" % (o, e) for o, e in f2m_lines])
+    f2m_block, f2m_dev_block = f2m_of(fuse), f2m_of(fuse_dev)
     if rel:
         coll, ma_names = _relative_collision_lines(spec)
     else:
         coll, ma_names = _collision_lines(spec, with_sources=True), mvars
-    b2 = _SumBuilder("r")
+    b2 = _SumBuilder("r", fuse)
     m2f_lines = _inverse_transform(b2, iM, ma_names, ["g%d" % k for k in range(ns)], ksym, sig_m2f)
     m2f_block = b2.lines + ["const C %s = %s;" % (o, e) for o, e in m2f_lines]
     stores = ["G%d[j] = Codec<S>::encode(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
     if rel:
         coll_dev, m2f_dev_block, stores_dev = coll, m2f_block, stores
     else:
-        coll_dev, dm_names = _deviation_collision_lines(spec)
-        bd = _SumBuilder("rd")
+        coll_dev, dm_names = _deviation_collision_lines(spec, fuse_dev)
+        bd = _SumBuilder("rd", fuse_dev)
         m2f_dev_lines = _inverse_transform(bd, iM, dm_names, ["g%d" % k for k in range(ns)], ksym, sig_m2f,
                                            tag="d")
         m2f_dev_block = bd.lines + ["const C %s = %s;" % (o, e) for o, e in m2f_dev_lines]
-        stores_dev = ["G%d[j] = Codec<S>::advance(L%d[j], f%d, g%d, a.wshift[%d]);" % (k, k, k, k, k) for k in range(ns)]
+        stores_dev = [("G%d[j] = Codec<S>::advance(L%d[j], f%d, g%d, a.wshift[%d]);" % (k, k, k, k, k)) if fuse_dev else
+                      ("G%d[j] = Codec<S>::encode_dev(f%d + g%d, a.wshift[%d]);" % (k, k, k, k)) for k in range(ns)]
 
     # ---------------------------------------------------------- f2m / m2f / eq
     b3 = _SumBuilder("p")
@@ -1654,7 +1677,8 @@ def generate_source(spec: KernelSpec) -> str:
             tb_mask=_indent(tb_mask, 8), tb_collect=_indent(tb_collect, 6), tb_entries=_indent(tb_entries), tb_apply=_indent(tb_apply, 4),
             tb_loads=_indent(tb_loads, 6), tb_sub=_indent(tb_sub, 6),
             tb_gdecl=_indent(["S %s;" % ", ".join("G%d[1]" % k for k in range(ns))], 6),
-            tb_coords=_indent(coords, 6), tb_decode=_indent(decode, 6), tb_f2m=_indent(f2m_block, 6),
+            tb_coords=_indent(coords, 6), tb_decode=_indent(decode, 6), tb_f2m=_indent(f2m_block, 8),
+            tb_f2m_dev=_indent(f2m_dev_block, 8),
             tb_coll_dev=_indent(coll_dev, 8), tb_m2f_dev=_indent(m2f_dev_block, 8),
             tb_stores_dev=_indent(stores_dev, 8), tb_coll=_indent(coll, 8), tb_m2f=_indent(m2f_block, 8),
             tb_stores=_indent(stores, 8),
@@ -1669,7 +1693,7 @@ def generate_source(spec: KernelSpec) -> str:
         vel=vel_txt,
         loads=_indent(loads), bbsub=_indent(bbsub), bbsub_ok=int(ksym is not None),
         gdecl=_indent(gdecl), coords=_indent(coords, 4), decode=_indent(decode, 4), vstores=_indent(vstores),
-        f2m=_indent(f2m_block, 4), coll=_indent(coll, 4), coll_dev=_indent(coll_dev, 4),
+        f2m=_indent(f2m_block, 4), f2m_dev=_indent(f2m_dev_block, 4), coll=_indent(coll, 4), coll_dev=_indent(coll_dev, 4),
         m2f=_indent(m2f_block, 4), m2f_dev=_indent(m2f_dev_block, 4), stores_dev=_indent(stores_dev, 4),
         stores=_indent(stores, 4),
         f2m_loads=_indent(f2m_loads), f2m_full=_indent(f2m_full), f2m_stores=_indent(f2m_stores),
