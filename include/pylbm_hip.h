@@ -285,6 +285,9 @@ typedef struct lbm_params {
    * 1 = one cell per thread, 4 = four (the contiguous interior extent must be a
    * multiple of 4); every choice gives the same bits */
   int32_t vec_cells;
+  /* lbm_gen_run on the wrap path: 0 = two steps per launch where that is the faster
+   * (3D), 1 = one step per launch; the same bits */
+  int32_t single_steps;
 } lbm_params;
 
 /* information on the generated module (ns, nconsm, dim) */

@@ -25,6 +25,7 @@ rows, printing/cython.py:347-349) is baked in.
 """
 import hashlib
 import os
+import re
 from fractions import Fraction
 
 import sympy as sp
@@ -499,6 +500,7 @@ using namespace lbm;
 #define TB_MASK %(bbsub_ok)d                    // folded links possible
 #define TB_BATCH 2                     // cells a thread of a blocked workgroup loads at once
 #define TB_LINKS 4                     // folded links a thread of a blocked workgroup holds
+#define PAIR_OK %(pair_ok)d            // the two-step kernel is generated
 
 namespace {
 
@@ -1057,8 +1059,23 @@ int lbm_gen_run(void* d_f, void* d_fnew, const lbm_layout* layout, const lbm_vel
   LBM_REQUIRE(!(periodic_fold && nmeth > 0), "periodic fold is only valid without link lists");
   void* a = d_f;
   void* b = d_fnew;
-  for (int64_t it = 0; it < nsteps; ++it) {
+  int64_t launches = 0;
+  for (int64_t it = 0; it < nsteps; ++it, ++launches) {
     int rc = 0;
+#if PAIR_OK
+    if (periodic_fold && it + 2 <= nsteps) {
+      bool done;
+      rc = pair_any(a, b, layout, params, &done, (hipStream_t)stream);
+      if (rc) return rc;
+      if (done) {
+        ++it;
+        void* tmp = a;
+        a = b;
+        b = tmp;
+        continue;
+      }
+    }
+#endif
     if (ghost == 1) rc = lbm_ghost_fill(a, layout, vel, stream);
     else if (ghost == 2) rc = lbm_ghost_fill_all(a, layout, vel, stream);
     if (rc) return rc;
@@ -1071,7 +1088,7 @@ int lbm_gen_run(void* d_f, void* d_fnew, const lbm_layout* layout, const lbm_vel
     b = tmp;
     params->t += params->dt;
   }
-  *parity = (int)(nsteps & 1);
+  *parity = (int)(launches & 1);
   return 0;
 }
 
@@ -1274,6 +1291,318 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
 
 """
 
+_PAIR_KERNEL = r"""// ------------------------------------------------ two steps per pass (3D)
+// A step of a grid past the caches is bound by HBM: it reads and writes every population
+// once.  This kernel advances two steps per read and write, with the per-cell arithmetic of
+// fused_step (the same generated lines, so the same bits), on the wrap path.  A workgroup
+// owns a column of 32 x ty cells (inner x mid axes) and walks along the outer axis.  For
+// each plane its threads, one per cell of the column and a halo of one cell around it, pull
+// and collide the first step into LDS; the column's own threads then do the second step
+// of the plane before, whose pulls from below, in and above are all there: two planes of
+// the upward populations, one of the level and one of the downward ones.  The next
+// plane's pulls are in flight meanwhile.  Folded bounce-back copies read the own cell
+// instead (MASK), in both steps.
+// 32 cells are 128 B of FP32; 13 rows and their halo are 510 of 512 threads, two
+// workgroups to a CU in 128 registers.  FP64 needs more registers (two workgroups: 75
+// spilled, 605 us per step of 150 x 201 x 183) and has a CU for one workgroup of 16 rows in
+// 168, with folded links 13 rows in 256.  What bounds it now: 256^3 FP32 at 306 us per step
+// moves 4.4 TB/s of HBM traffic (1.1 reads and 1 write per population and two steps) with
+// the vector units 43 %% busy; the rest are the barriers of two workgroups per CU.
+template <typename C>
+struct PairArgs {
+  int32_t tiles_i, tiles_m, ty, nz;   // tiles along the inner and mid axes, rows of a tile, planes per workgroup
+  C times[2];                     // t of each step
+};
+
+constexpr int PAIR_TX = 32, PAIR_RX = PAIR_TX + 2;
+
+template <typename S, bool MASK>
+constexpr int pair_rows() {
+  return sizeof(S) == 8 && !MASK ? 16 : 13;
+}
+template <int TY>
+constexpr int pair_threads() {
+  return ((TY + 2) * PAIR_RX + 63) / 64 * 64;
+}
+template <typename S, bool MASK, int TY>
+constexpr int pair_waves() {
+  return sizeof(S) == 8 ? (pair_threads<TY>() + 255) / 256 : 2 * pair_threads<TY>() / 256;
+}
+template <typename S, int TY>
+constexpr size_t pair_lds() {
+  return sizeof(S) * (2 * PAIR_UP + PAIR_LEVEL + PAIR_DOWN) * (TY + 2) * PAIR_RX;
+}
+
+__device__ __forceinline__ int pair_wrap(int x, int n) {
+  x += (x < 0) ? n : 0;
+  x -= (x >= n) ? n : 0;
+  x -= (x >= n) ? n : 0;
+  return x;
+}
+
+// a uniform value that the compiler must take as new in every pass of the loop: without
+// it the address of every population's slot is kept in two registers across the loop
+template <typename T>
+__device__ __forceinline__ T opaque(T x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
+// one plane of an array as a buffer: a load's address is the plane, a population's offset
+// in a scalar register and the column's in a vector register, without vector arithmetic
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p, uint64_t offset) {
+  return __builtin_amdgcn_make_buffer_rsrc((char*)const_cast<void*>(p) + offset, 0, 0xffffffffu, 0x00020000);
+}
+template <typename S>
+__device__ __forceinline__ S buffer_load(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
+  S x;
+  if constexpr (sizeof(S) == 8) {
+    const auto b = __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0);
+    __builtin_memcpy(&x, &b, 8);
+  } else {
+    const auto b = __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0);
+    __builtin_memcpy(&x, &b, 4);
+  }
+  return x;
+}
+// non-temporal (aux bit 1), as the population stores of fused_step
+template <typename S>
+__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s, S x) {
+  if constexpr (sizeof(S) == 8) {
+    typedef uint32_t v2 __attribute__((ext_vector_type(2)));
+    v2 b;
+    __builtin_memcpy(&b, &x, 8);
+    __builtin_amdgcn_raw_buffer_store_b64(b, r, v, s, LBM_NT_STORES ? 2 : 0);
+  } else {
+    uint32_t b;
+    __builtin_memcpy(&b, &x, 4);
+    __builtin_amdgcn_raw_buffer_store_b32(b, r, v, s, LBM_NT_STORES ? 2 : 0);
+  }
+}
+
+// the value of a load, waited for here
+template <typename S>
+__device__ __forceinline__ S arrived(S x) {
+  typename Bits<S>::T b;
+  __builtin_memcpy(&b, &x, sizeof(S));
+  asm volatile("" : "+v"(b));
+  __builtin_memcpy(&x, &b, sizeof(S));
+  return x;
+}
+
+// the collision of fused_step for one cell (the same generated lines, so the same bits)
+template <typename S>
+__device__ __forceinline__ void pair_collide(const S (&L)[NS], S (&G)[NS],
+                                             const StepArgs<typename Codec<S>::C>& a, int o, int m, int ii,
+                                             typename Codec<S>::C tt) {
+  using C = typename Codec<S>::C;
+  constexpr bool DEV = Codec<S>::kind != LBM_F64;
+  constexpr int j = 0;
+  const C half_dt = a.half_dt;
+  const C* one_minus = a.one_minus;
+  const C* omega = a.omega;
+  const C* cref = a.cref;
+  (void)half_dt; (void)tt; (void)cref; (void)j; (void)o; (void)m; (void)ii; (void)one_minus; (void)omega;
+%(pair_coords)s
+%(pair_decode)s
+  if constexpr (DEV) {
+%(pair_f2m_dev)s
+%(pair_coll_dev)s
+%(pair_m2f_dev)s
+%(pair_stores_dev)s
+  } else {
+%(pair_f2m)s
+%(pair_coll)s
+%(pair_m2f)s
+%(pair_stores)s
+  }
+}
+
+template <typename S, bool MASK, int TY>
+__global__ void __launch_bounds__(pair_threads<TY>()) __attribute__((amdgpu_waves_per_eu(pair_waves<S, MASK, TY>())))
+pair_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Codec<S>::C> a,
+          const PairArgs<typename Codec<S>::C> t) {
+  constexpr int RX = PAIR_RX, RY = TY + 2, R = RX * RY;
+  extern __shared__ double pair_smem[];
+  S* const up = reinterpret_cast<S*>(pair_smem);   // [2][PAIR_UP][R]
+  S* const level = up + 2 * PAIR_UP * R;           // [PAIR_LEVEL][R]
+  S* const down = level + PAIR_LEVEL * R;          // [PAIR_DOWN][R]
+  const int total = gridDim.x, xcd = blockIdx.x %% 8;
+  const int lin = xcd * (total / 8) + min(xcd, total %% 8) + (int)blockIdx.x / 8;
+  const int i0 = lin %% t.tiles_i * PAIR_TX, m0 = lin / t.tiles_i %% t.tiles_m * t.ty;
+  const int z0 = lin / (t.tiles_i * t.tiles_m) * t.nz, z1 = min(z0 + t.nz, a.nin[0]);
+  const int c = threadIdx.x, e = c - RY * PAIR_TX;
+  const int ry = min(e < 0 ? c / PAIR_TX : e >> 1, t.ty + 1);   // the threads past the last row repeat it
+  const bool active = c < R;
+  const int rx = e < 0 ? 1 + c %% PAIR_TX : (e & 1) * (RX - 1);
+  const int at = ry * RX + rx;
+  const int gm = pair_wrap(m0 - 1 + ry, a.nin[1]), gi = pair_wrap(i0 - 1 + rx, a.nin[2]);
+  const bool owner = e < 0 && ry >= 1 && ry <= t.ty && m0 + ry <= a.nin[1] && i0 + rx <= a.nin[2];
+  const uint64_t plane = (uint64_t)a.n1 * a.rs * sizeof(S);
+  const uint32_t pop = NS > 1 ? (uint32_t)(a.dst_off[1] * sizeof(S)) : 0u;
+  // byte offsets inside one plane of one population, of the cell and the cells it pulls from
+%(pair_lat)s
+  const uint32_t* const mask = MASK ? a.bbmask + (int64_t)gm * a.nin[2] + gi : nullptr;
+  const int64_t mplane = (int64_t)a.nin[1] * a.nin[2];
+  S P[NS];
+  const auto fetch = [&](int p, uint32_t bits) {
+    const int op = pair_wrap(p, a.nin[0]);
+    const uint64_t z_0 = (op + a.halo[0]) * plane;
+    const uint64_t z_p1 = (pair_wrap(op - 1, a.nin[0]) + a.halo[0]) * plane;
+    const uint64_t z_n1 = (pair_wrap(op + 1, a.nin[0]) + a.halo[0]) * plane;
+    const auto r_0 = buffer(f, z_0), r_p1 = buffer(f, z_p1), r_n1 = buffer(f, z_n1), r_f = buffer(f, 0);
+    uint32_t kb = opaque(0u);
+    (void)z_0; (void)z_p1; (void)z_n1;
+    if (MASK && __ballot(bits != 0)) {
+%(pair_fetch_mask)s
+    } else {
+%(pair_fetch)s
+    }
+  };
+  const auto maskword = [&](int p) { return mask[pair_wrap(p, a.nin[0]) * mplane]; };
+  uint32_t b_p = 0, b_c = 0, b_n = 0;   // mask words of planes p - 1, p, p + 1
+  if (MASK) {
+    b_c = maskword(z0 - 1);
+    b_n = maskword(z0);
+  }
+  fetch(z0 - 1, b_c);
+  for (int p = z0 - 1; p <= z1; ++p) {
+    S L[NS], G[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) L[k] = P[k];
+    uint32_t b_nn = 0;
+    if (p < z1) {
+      fetch(p + 1, b_n);
+      if (MASK && p + 1 < z1) b_nn = maskword(p + 2);
+    }
+    pair_collide<S>(L, G, a, pair_wrap(p, a.nin[0]) + a.halo[0], gm + a.halo[1], gi + a.halo[2], t.times[0]);
+    // the second step at plane p - 1: what lies below it and in it
+    const bool second = p > z0 && owner;
+    S* const up_p = up + (p & 1) * PAIR_UP * R;
+    const S* const up_1 = up + (p & 1 ^ 1) * PAIR_UP * R;
+    (void)up_1;
+    if (second) {
+%(pair_read1)s
+    }
+    __syncthreads();
+    if (active) {
+%(pair_write)s
+    }
+    __syncthreads();
+    if (second) {
+%(pair_read2)s
+      pair_collide<S>(L, G, a, p - 1 + a.halo[0], gm + a.halo[1], gi + a.halo[2], t.times[1]);
+    }
+    // the next plane is waited for before the stores: behind them the wait would be for
+    // the stores as well
+#pragma unroll
+    for (int k = 0; k < NS; ++k) P[k] = arrived(P[k]);
+    if (second) {
+      const auto r_out = buffer(fn, (p - 1 + a.halo[0]) * plane);
+      uint32_t kb = opaque(0u);
+%(pair_store)s
+    }
+    if (MASK) {
+      b_p = b_c;
+      b_c = b_n;
+      b_n = b_nn;
+    }
+  }
+  (void)b_p;
+}
+
+"""
+
+_PAIR_LAUNCH = r"""template <typename S, bool MASK>
+static int pair_launch(const void* f, void* fn, const lbm_layout* L, lbm_params* p, int nz, hipStream_t s) {
+  using C = typename Codec<S>::C;
+  constexpr int TY = pair_rows<S, MASK>();
+  StepArgs<C> a;
+  int rc = make_args<C>(L, p, &a);
+  if (rc) return rc;
+  PairArgs<C> t{};
+  t.tiles_i = (a.nin[2] + PAIR_TX - 1) / PAIR_TX;
+  t.tiles_m = (a.nin[1] + TY - 1) / TY;
+  t.ty = (a.nin[1] + t.tiles_m - 1) / t.tiles_m;
+  t.nz = nz;
+  for (int q = 0; q < 2; ++q) {
+    t.times[q] = (C)p->t;
+    p->t += p->dt;
+  }
+  const size_t lds = pair_lds<S, TY>();
+  const unsigned groups = (unsigned)(t.tiles_i * t.tiles_m * ((a.nin[0] + nz - 1) / nz));
+  const auto kernel = pair_step<S, MASK, TY>;
+  if (lds > 64 * 1024)
+    LBM_CHECK_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  kernel<<<groups, pair_threads<TY>(), lds, s>>>((const S*)f, (S*)fn, a, t);
+  LBM_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+
+// Planes per workgroup of the two-step kernel on this grid, or 0: one step at a time.
+// The choice is between whole runs of one step per launch at 5.6 TB/s of reads and writes
+// plus 2 us, and the least estimate of the two-step kernel over the numbers of chunks
+// along the outer axis: nz + 2 planes per workgroup at so many us per plane with few
+// workgroups, one or two on every CU, a little more in long chunks, whose neighbours
+// drift apart in the L2 (constants fitted to a sweep of 19 grids, 80^3 to 256^3, with and
+// without folded links, FP32 and FP64 D3Q19 on MI355X: 5 % rms).  Per step, one at a time /
+// two: 256^3 FP32 452 / 306 us, 128^3 59 / 47, 80^3 18 / 19; 150 x 201 x 183 FP64 310 / 205,
+// 80^3 31 / 24; 256 x 128 x 128 with spheres FP32 117 / 99, FP64 222 / 170.
+template <typename S, bool MASK>
+static int pair_planes(const int32_t (&nin)[3]) {
+  constexpr double part = NS / 19.0;
+  constexpr double few = part * (sizeof(S) == 8 ? (MASK ? 4.3 : 4.9) : 2.9);
+  constexpr double one = part * (sizeof(S) == 8 ? (MASK ? 6.6 : 7.7) : 4.1), two = part * 7.0;
+  constexpr double drift = MASK ? 0.006 : 0.0008, start = MASK ? 5.0 : 1.0;
+  const int64_t tiles = (int64_t)((nin[2] + PAIR_TX - 1) / PAIR_TX) *
+                        ((nin[1] + pair_rows<S, MASK>() - 1) / pair_rows<S, MASK>());
+  double best = 0.9 * 2.0 * (2.0 + (double)nin[0] * nin[1] * nin[2] * NS * 2.0 * sizeof(S) / 5.6e6);
+  int planes = 0;
+  for (int chunks = 1; chunks <= nin[0] / 4; ++chunks) {
+    const int nz = (nin[0] + chunks - 1) / chunks;
+    const int64_t groups = tiles * ((nin[0] + nz - 1) / nz), cap = sizeof(S) == 8 ? 256 : 512;
+    const int64_t rest = groups %% cap;
+    double us = (double)(groups / cap) * (sizeof(S) == 8 ? one : two);
+    if (rest > 256) us += two * (0.85 + 0.15 * (double)(rest - 256) / 256.0);
+    else if (rest > 0) us += few + (one - few) * (double)rest / 256.0;
+    us = start + (nz + 2) * (1.0 + drift * nz) * us;
+    if (us < best) {
+      best = us;
+      planes = nz;
+    }
+  }
+  return planes;
+}
+
+// one launch of the two-step kernel, where it is the faster one (*done)
+template <typename S, bool MASK>
+static int pair_try(const void* f, void* fn, const lbm_layout* L, lbm_params* p, bool* done, hipStream_t s) {
+  // an offset inside a plane (with folded links inside the array) is below 2^31 bytes
+  const int64_t reach = ((NS - 1) * L->pop_stride + (MASK ? L->n[0] : 1) * L->n[1] * L->row_stride) * (int64_t)sizeof(S);
+  int32_t nin[3];
+  for (int d = 0; d < 3; ++d) nin[d] = (int32_t)(L->n[d] - 2 * L->halo[d]);
+  if (pair_lds<S, pair_rows<S, MASK>()>() > 160 * 1024 || reach >= (int64_t)1 << 31 || nin[0] < 4 || nin[1] < 32 || nin[2] < 32) return 0;
+  const int nz = pair_planes<S, MASK>(nin);
+  if (nz == 0) return 0;
+  *done = true;
+  return pair_launch<S, MASK>(f, fn, L, p, nz, s);
+}
+
+static int pair_any(const void* f, void* fn, const lbm_layout* L, lbm_params* p, bool* done, hipStream_t s) {
+  *done = false;
+  // folded links beyond copies (a table), a launch shape asked for, or 2-byte formats (bound
+  // by arithmetic: 128^3 FP16 33 us per step one at a time, 40 us in pairs): single steps
+  if (p->bbtab_bits || p->vec_cells != 0 || p->xcd_remap >= 0 || p->single_steps) return 0;
+  switch (L->storage) {
+    case LBM_F64: return p->bbmask ? pair_try<double, true>(f, fn, L, p, done, s) : pair_try<double, false>(f, fn, L, p, done, s);
+    case LBM_F32: return p->bbmask ? pair_try<float, true>(f, fn, L, p, done, s) : pair_try<float, false>(f, fn, L, p, done, s);
+    case LBM_F32D: return p->bbmask ? pair_try<f32dev, true>(f, fn, L, p, done, s) : pair_try<f32dev, false>(f, fn, L, p, done, s);
+  }
+  return 0;
+}
+
+"""
+
 _TB_LAUNCH = r"""// one launch of tb_step: nt steps of every tile; advances params->t by nt dt
 template <typename S>
 static int tb_launch(void* f, void* fn, const lbm_layout* L, lbm_params* p, int nt, int tm, int ti,
@@ -1339,6 +1668,71 @@ _TB_LAUNCH_NONE = r"""#define LBM_DISPATCH_BLOCKED(kind, FN, f, fn, L, p, nt, tm
   } while (0)
 
 """
+
+
+def _pair_source(vel, ksym, decode, coords, f2m, f2m_dev, coll_dev, m2f_dev, stores_dev, coll, m2f, stores):
+    """The kernel that advances a 3D scheme with velocity components in {-1, 0, 1} by two
+    steps per pass over memory."""
+    ns = len(vel)
+    arr = lambda lines: [re.sub(r"\b([LG])(\d+)\[j\]", r"\1[\2]", ln) for ln in lines]   # noqa: E731
+    nm = lambda c: ("p%d" % c) if c > 0 else ("n%d" % -c if c < 0 else "0")   # noqa: E731
+    slot = {}
+    for name, v0 in (("up", 1), ("level", 0), ("down", -1)):
+        ks = [k for k in range(ns) if vel[k][0] == v0]
+        slot.update({k: (name, q) for q, k in enumerate(ks)})
+    count = {n: max([q + 1 for m, q in slot.values() if m == n], default=0) for n in ("up", "level", "down")}
+    lat = []
+    for d, axis, n, step in ((1, "gm", 1, "(uint32_t)a.rs"), (2, "gi", 2, "1u")):
+        for c in sorted({v[d] for v in vel} | {0}):
+            extra = " + (uint32_t)(a.lead + a.halo[2])" if d == 2 else ""
+            halo = " + a.halo[1]" if d == 1 else ""
+            lat.append("  const uint32_t s%d_%s = ((uint32_t)(pair_wrap(%s - (%d), a.nin[%d])%s) * %s%s) * (uint32_t)sizeof(S);"
+                       % (d, nm(c), axis, c, n, halo, step, extra))
+    offs = sorted({v[1:] for v in vel} | {(0, 0)})
+    lat += ["  const uint32_t o_%s_%s = s1_%s + s2_%s;" % (nm(a), nm(b), nm(a), nm(b)) for a, b in offs]
+    ref = lambda k: "o_%s_%s" % (nm(vel[k][1]), nm(vel[k][2]))   # noqa: E731
+    # kb runs over the populations (opaque: the compiler would multiply again for each)
+    fetch, fetch_mask = [], []
+    for k in range(ns):
+        step = "" if k == 0 else "      kb = opaque(kb + pop);\n"
+        load = "      P[%d] = buffer_load<S>(r_%s, %s, kb);" % (k, nm(vel[k][0]), ref(k))
+        fetch.append(step + load)
+        if ksym is not None and ksym[k] != k:
+            fetch_mask.append(step + "      P[%d] = buffer_load<S>(r_f, (bits & %du) ? o_0_0 + (%du * pop + (uint32_t)z_0) :"
+                              " %s + (kb + (uint32_t)z_%s), 0u); __builtin_amdgcn_sched_barrier(0);"
+                              % (k, 1 << k, ksym[k], ref(k), nm(vel[k][0])))
+        else:
+            fetch_mask.append(step + load)
+    read1, write, read2, store = [], [], [], []
+    for k in range(ns):
+        name, q = slot[k]
+        near = "[%d * R + at - (%d)]" % (q, vel[k][1] * 34 + vel[k][2])
+        write.append("      %s[%d * R + at] = G[%d];" % ("up_p" if name == "up" else name, q, k))
+        bounce = ksym is not None and ksym[k] != k
+        if bounce:
+            # population ksym at the own cell after the first step: planes p - 1 of LDS,
+            # before plane p is written
+            oname, oq = slot[ksym[k]]
+            own = "%s[%d * R + at]" % ("up_1" if oname == "up" else oname, oq)
+        if name == "down":
+            if bounce:
+                read1.append("      if (MASK && (b_p & %du)) L[%d] = %s;" % (1 << k, k, own))
+            read2.append("      %sL[%d] = down%s;" % ("if (!MASK || !(b_p & %du)) " % (1 << k) if bounce else "", k, near))
+        else:
+            x = ("up_p" if name == "up" else name) + near
+            read1.append("      L[%d] = %s%s;" % (k, "(MASK && (b_p & %du)) ? %s : " % (1 << k, own) if bounce else "", x))
+    for k in range(ns):
+        store.append("      buffer_store<S>(r_out, o_0_0, kb, G[%d]);" % k
+                     + (" kb = opaque(kb + pop);" if k < ns - 1 else ""))
+    j = "\n".join
+    return (_PAIR_KERNEL % dict(
+        pair_coords=_indent(coords), pair_decode=_indent(arr(decode)), pair_f2m=_indent(f2m, 4), pair_f2m_dev=_indent(f2m_dev, 4),
+        pair_coll_dev=_indent(coll_dev, 4), pair_m2f_dev=_indent(m2f_dev, 4), pair_stores_dev=_indent(arr(stores_dev), 4),
+        pair_coll=_indent(coll, 4), pair_m2f=_indent(m2f, 4), pair_stores=_indent(arr(stores), 4),
+        pair_lat=j(lat), pair_fetch_mask=j(fetch_mask), pair_fetch=j(fetch), pair_read1=j(read1),
+        pair_write=j(write), pair_read2=j(read2), pair_store=j(store))
+        ).replace("PAIR_UP", str(count["up"])).replace("PAIR_LEVEL", str(count["level"])).replace(
+            "PAIR_DOWN", str(count["down"]))
 
 
 def _indent(lines, n=2):
@@ -1687,8 +2081,13 @@ def generate_source(spec: KernelSpec) -> str:
     else:
         tb_kernel = ""
         tb_launch = _TB_LAUNCH_NONE
+        # up to D3Q19: what a thread holds of more populations does not fit its registers
+        if ns <= 19 and not rel and all(abs(c) <= 1 for v in vel for c in v):
+            tb_launch = _PAIR_LAUNCH % {} + _TB_LAUNCH_NONE
+            tb_kernel = _pair_source(vel, ksym, decode, coords, f2m_block, f2m_dev_block, coll_dev, m2f_dev_block, stores_dev, coll,
+                                     m2f_block, stores)
     return _TEMPLATE % dict(
-        tb_kernel=tb_kernel, tb_launch=tb_launch, unit_vel=int(all(abs(c) <= 1 for v in vel for c in v)),
+        tb_kernel=tb_kernel, tb_launch=tb_launch, pair_ok=int(dim == 3 and bool(tb_kernel)), unit_vel=int(all(abs(c) <= 1 for v in vel for c in v)),
         hash=spec_hash(spec), ns=ns, nc=spec.nconsm, dim=dim, paired=bool(sig_f2m),
         vel=vel_txt,
         loads=_indent(loads), bbsub=_indent(bbsub), bbsub_ok=int(ksym is not None),

@@ -258,8 +258,8 @@ class Simulation:
         # bounce-back / anti-bounce-back lists folded into the fused step's pulls when
         # that is exact (False: every list runs as a link-list launch; same results)
         self.fold_links = True
-        # small 2D grids on the wrap path advance several steps per launch in LDS
-        # (run() only; same results, see _blocking_shape)
+        # 1D and 2D grids on the wrap path advance several steps per launch in LDS (see
+        # _blocking_shape), 3D grids two (run() only; same results)
         self.temporal_blocking = True
         self.init_type = dico.get("inittype", "moments")
         self.init_data = dico.get("init", None)
@@ -806,6 +806,7 @@ class Simulation:
             self.nt += nsteps
             self.t = self.t + nsteps * self.dt
             return
+        self.params.single_steps = 0 if self.temporal_blocking else 1
         ghost = 0 if fold else self._ghost_mode
         nmeth = 0 if fold else len(self._active_links)
         self._check(self.module.lbm_gen_run(ctypes.c_void_p(c.F.ptr), ctypes.c_void_p(c.Fnew.ptr),
