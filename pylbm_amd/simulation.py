@@ -42,8 +42,12 @@ __all__ = ["Simulation"]
 LBM_F64 = rtm.LBM_F64
 # Largest table (links that are not a copy of the cell's own ksym population) the
 # whole-step fold may build: table entries are scattered reads inside the step's
-# waves, and 126,620 of them spread over C4's waves cost 37 us per step against a
-# 4.5 us launch of the same copies (MI355X); smaller tables save their launches.
+# waves, and 126,620 of them spread over the waves of a 512 x 256 x 256 sphere packing
+# cost 37 us per step against a 4.5 us launch of the same copies (MI355X); smaller tables
+# save their launches.  With Neumann lists, which fold in no other way, the table takes
+# the place of the ghost fill and every launch, and is four times as large: 240 x 112 x 112
+# duct, 125,440 entries on its inflow and outflow faces, FP32 118 us per step in launches,
+# 93 us folded; FP64 198 and 159.
 FOLD_TABLE_MAX = 1 << 16
 # Temporally blocked run in 1D: (steps per launch, cells per tile); a tile and its halo
 # of steps cells on both sides fill one region of TB_PLANE_1D cells (the generated
@@ -455,7 +459,8 @@ class Simulation:
         ksym = np.asarray(self.scheme.stencil.get_symmetric())[k]
         own = ksym * L.pop_stride + (x[0] * L.n[1] + x[1]) * L.row_stride + L.lead + x[2]
         copy = (org == own) & (sg == 1.0) & ~has & (org2 < 0)
-        if np.count_nonzero(~copy) > FOLD_TABLE_MAX:
+        neumann = any(not isinstance(d.method, str) and d.method.kind.name.startswith("neumann") for d in devs)
+        if np.count_nonzero(~copy) > FOLD_TABLE_MAX * (4 if neumann else 1):
             return False
         mask = np.zeros(int(np.prod(nin)), dtype=np.uint32)
         np.bitwise_or.at(mask, cell, np.uint32(1) << k.astype(np.uint32))
