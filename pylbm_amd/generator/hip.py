@@ -478,11 +478,12 @@ def _equilibrium_lines(spec: KernelSpec):
 # ------------------------------------------------------------------ template
 _TEMPLATE = r"""// Generated by pylbm_amd.generator.hip for scheme %(hash)s -- do not edit.
 // ns=%(ns)d nconsm=%(nc)d dim=%(dim)d pair-factored=%(paired)s
-// Population stores bypass the caches (each value is read once, in the next step).
+// Population stores may bypass the caches (stream_stores).
 #ifndef LBM_NT_STORES
 #define LBM_NT_STORES 1
 #endif
 #include "lbm_device.h"
+#include <type_traits>
 
 using namespace lbm;
 
@@ -512,6 +513,7 @@ struct StepArgs {
   int32_t halo[3];
   int32_t n1, rs, lead, remap;     // rs: elements between consecutive rows; remap: XCD-aware order
   int32_t ends_first;              // planes from both ends to the middle
+  int32_t nt;                      // population stores past the caches
   const uint32_t* bbmask;          // NULL or folded link directions per interior cell
   const uint32_t* bbtab_bits;      // NULL or the folded links with a sign / value table entry
   const uint32_t* bbtab_base;
@@ -586,6 +588,30 @@ __device__ __forceinline__ void block_coords(unsigned& bx, unsigned& by, unsigne
       by = (logical / gridDim.x) %% gridDim.y;
       bz = logical / (gridDim.x * gridDim.y);
     }
+  }
+}
+
+// memory from an offset of an array on as a buffer: an address is its start, an offset in a
+// scalar register and one in a vector register (32 bits each), without vector arithmetic
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p, uint64_t offset) {
+  return __builtin_amdgcn_make_buffer_rsrc((char*)const_cast<void*>(p) + offset, 0, 0xffffffffu, 0x00020000);
+}
+// non-temporal (aux bit 1) or not
+template <typename S, bool NT>
+__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s, S x) {
+  if constexpr (sizeof(S) == 8) {
+    typedef uint32_t v2 __attribute__((ext_vector_type(2)));
+    v2 b;
+    __builtin_memcpy(&b, &x, 8);
+    __builtin_amdgcn_raw_buffer_store_b64(b, r, v, s, NT ? 2 : 0);
+  } else if constexpr (sizeof(S) == 4) {
+    uint32_t b;
+    __builtin_memcpy(&b, &x, 4);
+    __builtin_amdgcn_raw_buffer_store_b32(b, r, v, s, NT ? 2 : 0);
+  } else {
+    uint16_t b;
+    __builtin_memcpy(&b, &x, 2);
+    __builtin_amdgcn_raw_buffer_store_b16(b, r, v, s, NT ? 2 : 0);
   }
 }
 
@@ -771,6 +797,16 @@ eq_m2f_kernel(const double* __restrict__ mo, lbm_layout ml, S* __restrict__ f, l
 %(m2f_stores)s
 }
 
+// Population stores bypass the caches, unless both arrays together are 24 to 320 MB: the
+// next step then finds them in the 256 MB Infinity Cache (us per step of D3Q19, past /
+// into the caches: 64^3 FP32 10.2 / 8.7, FP64 18.1 / 14.7, 96^3 FP32 26.2 / 23.4, 128^3 FP32
+// (319 MB) 59 / 54; 128^3 FP64 (637 MB) 113 / 125, 160^3 FP32 106 / 118).  Small grids wait
+// for the L2s to be written back at the end of every step (64^2 FP64 4.7 / 5.6).
+static int stream_stores(const lbm_layout* L) {
+  const int64_t bytes = 2 * L->n[0] * L->n[1] * L->pitch * L->ns * (int64_t)storage_elem_size(L->storage);
+  return bytes < (int64_t)24 << 20 || bytes > (int64_t)320 << 20;
+}
+
 template <typename C>
 static int make_args(const lbm_layout* L, const lbm_params* p, StepArgs<C>* a) {
   int rc = check_layout(L);
@@ -790,6 +826,7 @@ static int make_args(const lbm_layout* L, const lbm_params* p, StepArgs<C>* a) {
   a->lead = (int32_t)L->lead;
   a->remap = 0;
   a->ends_first = 0;
+  a->nt = stream_stores(L);
   for (int k = 0; k < NS; ++k) {
     a->omega[k] = p ? (C)p->omega[k] : (C)0;
     a->one_minus[k] = p ? (C)p->one_minus[k] : (C)1;
@@ -1353,11 +1390,6 @@ __device__ __forceinline__ T opaque(T x) {
   return x;
 }
 
-// one plane of an array as a buffer: a load's address is the plane, a population's offset
-// in a scalar register and the column's in a vector register, without vector arithmetic
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p, uint64_t offset) {
-  return __builtin_amdgcn_make_buffer_rsrc((char*)const_cast<void*>(p) + offset, 0, 0xffffffffu, 0x00020000);
-}
 template <typename S>
 __device__ __forceinline__ S buffer_load(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
   S x;
@@ -1370,21 +1402,6 @@ __device__ __forceinline__ S buffer_load(__amdgpu_buffer_rsrc_t r, uint32_t v, u
   }
   return x;
 }
-// non-temporal (aux bit 1), as the population stores of fused_step
-template <typename S>
-__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s, S x) {
-  if constexpr (sizeof(S) == 8) {
-    typedef uint32_t v2 __attribute__((ext_vector_type(2)));
-    v2 b;
-    __builtin_memcpy(&b, &x, 8);
-    __builtin_amdgcn_raw_buffer_store_b64(b, r, v, s, LBM_NT_STORES ? 2 : 0);
-  } else {
-    uint32_t b;
-    __builtin_memcpy(&b, &x, 4);
-    __builtin_amdgcn_raw_buffer_store_b32(b, r, v, s, LBM_NT_STORES ? 2 : 0);
-  }
-}
-
 // the value of a load, waited for here
 template <typename S>
 __device__ __forceinline__ S arrived(S x) {
@@ -1504,8 +1521,13 @@ pair_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename C
     for (int k = 0; k < NS; ++k) P[k] = arrived(P[k]);
     if (second) {
       const auto r_out = buffer(fn, (p - 1 + a.halo[0]) * plane);
-      uint32_t kb = opaque(0u);
+      const auto store = [&](auto nt) {
+        constexpr bool NT = decltype(nt)::value;
+        uint32_t kb = opaque(0u);
 %(pair_store)s
+      };
+      if (a.nt) store(std::true_type{});
+      else store(std::false_type{});
     }
     if (MASK) {
       b_p = b_c;
@@ -1582,11 +1604,11 @@ static int pair_planes(const int32_t (&nin)[3]) {
 // one launch of the two-step kernel, where it is the faster one (*done)
 template <typename S, bool MASK>
 static int pair_try(const void* f, void* fn, const lbm_layout* L, lbm_params* p, bool* done, hipStream_t s) {
-  // an offset inside a plane (with folded links inside the array) is below 2^31 bytes
+  // an offset inside a plane (with folded links inside the array) has 32 bits
   const int64_t reach = ((NS - 1) * L->pop_stride + (MASK ? L->n[0] : 1) * L->n[1] * L->row_stride) * (int64_t)sizeof(S);
   int32_t nin[3];
   for (int d = 0; d < 3; ++d) nin[d] = (int32_t)(L->n[d] - 2 * L->halo[d]);
-  if (pair_lds<S, pair_rows<S, MASK>()>() > 160 * 1024 || reach >= (int64_t)1 << 31 || nin[0] < 4 || nin[1] < 32 || nin[2] < 32) return 0;
+  if (pair_lds<S, pair_rows<S, MASK>()>() > 160 * 1024 || reach >= ((int64_t)1 << 32) - (1 << 20) || nin[0] < 4 || nin[1] < 32 || nin[2] < 32) return 0;
   const int nz = pair_planes<S, MASK>(nin);
   if (nz == 0) return 0;
   *done = true;
@@ -1727,7 +1749,7 @@ def _pair_source(vel, ksym, decode, coords, f2m, f2m_dev, coll_dev, m2f_dev, sto
             x = ("up_p" if name == "up" else name) + near
             read1.append("      L[%d] = %s%s;" % (k, "(MASK && (b_p & %du)) ? %s : " % (1 << k, own) if bounce else "", x))
     for k in range(ns):
-        store.append("      buffer_store<S>(r_out, o_0_0, kb, G[%d]);" % k
+        store.append("        buffer_store<S, NT>(r_out, o_0_0, kb, G[%d]);" % k
                      + (" kb = opaque(kb + pop);" if k < ns - 1 else ""))
     j = "\n".join
     return (_PAIR_KERNEL % dict(
@@ -1870,6 +1892,10 @@ def generate_source(spec: KernelSpec) -> str:
         decode = ["C f%d = DEV ? Codec<S>::decode_dev(L%d[j], a.wshift[%d]) : Codec<S>::decode(L%d[j], a.wshift[%d]);"
                   % (k, k, k, k, k) for k in range(ns)]
     vstores = ["vstore<S, VEC>(fn + ((I)a.dst_off[%d] + cell), G%d);" % (k, k) for k in range(ns)]
+    cstores = ["buffer_store<S, false>(r_, (uint32_t)(cell * sizeof(S)), (uint32_t)(a.dst_off[%d] * sizeof(S)), G%d[0]);"
+               % (k, k) for k in range(ns)]
+    vstores = (["if (VEC > 1 || sizeof(I) > 4 || a.nt) {"] + ["  " + ln for ln in vstores] + ["} else {", "  const auto r_ = buffer(fn, 0);"]
+               + ["  " + ln for ln in cstores] + ["}"])
 
     # The arithmetic of the step.  With fuse (FP64, and every format in 3D) moments share
     # partial sums and products are contracted: a quarter fewer instructions.  The

@@ -1,6 +1,7 @@
 """3D boxes with inflow values and outflow copies fold into the step with a table on two
 faces (batches of entries, planes taken from both ends): the bits of the link launches,
-for extents with an even and an odd number of planes and a single plane between the faces."""
+for extents with an even and an odd number of planes and a single plane between the faces.
+Stores into the caches (24 to 320 MB of populations) give the bits of stores past them."""
 import numpy as np
 import pytest
 
@@ -46,5 +47,17 @@ def test_duct_fold_equals_launches(hip, shape, axis, dtype):
         _noise(sim)
         sim.one_time_step()
         sim.run(7)
+    for k in range(a.ns):
+        assert np.array_equal(a.F[k], b.F[k]), k
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+def test_cached_stores(hip, dtype):
+    d = cases.taylor_green_d3q19(96)   # 269 MB in FP64: past / into the caches by format
+    a, b = Simulation(d, dtype=dtype), Simulation(d, dtype=dtype)
+    b.params.vec_cells = 4             # four cells per thread, always past the caches
+    for sim in (a, b):
+        sim.run(3)
+        sim.one_time_step()
     for k in range(a.ns):
         assert np.array_equal(a.F[k], b.F[k]), k
