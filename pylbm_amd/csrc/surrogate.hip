@@ -707,13 +707,16 @@ __global__ void __launch_bounds__(256) sum_partials_kernel(const float* __restri
   if (wv == 0 && i < n) dst[i] = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
 }
 
-// Masked mean-square loss over the 48 value channels of 64; dY = 2 gscale (y - t) as E
+// Masked mean-square loss over the 48 value channels of 64; dY = 2 gscale (y - t) as E.
+// Bound by its 84 MB (8 x 128 x 128 pixels); 256 partial sums, so one workgroup per CU,
+// which needs all its 16 waves to have enough loads in flight
+constexpr int MSE_THREADS = 1024;
 template <typename E>
-__global__ void __launch_bounds__(256) mse_kernel(const float* __restrict__ y, const float* __restrict__ tg,
+__global__ void __launch_bounds__(MSE_THREADS) mse_kernel(const float* __restrict__ y, const float* __restrict__ tg,
                                                   int64_t nq, float gscale, E* __restrict__ dy,
                                                   double* __restrict__ partial) {
   typedef typename Elem<E>::v4 half4;
-  __shared__ double sh[256];
+  __shared__ double sh[MSE_THREADS];
   double s = 0.0;
   // one float4 = the 4 fields of one fine pixel; field 3 carries nothing
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nq; i += (int64_t)gridDim.x * blockDim.x) {
@@ -731,7 +734,7 @@ __global__ void __launch_bounds__(256) mse_kernel(const float* __restrict__ y, c
   }
   sh[threadIdx.x] = s;
   __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
+  for (int off = MSE_THREADS / 2; off > 0; off >>= 1) {
     if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
     __syncthreads();
   }
@@ -1254,7 +1257,7 @@ int lbm_sur_mse(const float* d_y, const float* d_t, int64_t npix, float gscale, 
   const int64_t nq = npix * 16;  // fine pixels
   const int rc = with_elem(elem, "mse", [&](auto tag) -> int {
     using E = typename decltype(tag)::type;
-    mse_kernel<E><<<256, 256, 0, s>>>(d_y, d_t, nq, gscale, (E*)d_dy, d_partial);
+    mse_kernel<E><<<256, MSE_THREADS, 0, s>>>(d_y, d_t, nq, gscale, (E*)d_dy, d_partial);
     return 0;
   });
   if (rc) return rc;
