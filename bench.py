@@ -1,15 +1,15 @@
 """Benchmark: D3Q19 MRT Taylor-Green vortex, 256^3 cells, FP32 populations, one MI355X.
 
 A step is one ``Simulation.one_time_step`` pass of the hot path over the
-256^3 periodic box (for this fully periodic box the fused pull/collide kernel
-reads through the periodic wrap, so a step is exactly one kernel launch).
+256^3 periodic box (for this fully periodic box the pull/collide kernel reads
+through the periodic wrap and advances two steps per launch).
 The timed region starts with the populations resident in HBM: W warm-up steps,
 device sync, K timed steps between HIP events on the simulation's stream,
 device sync.  Printed as one JSON line:
 
   value     MLUPS = cells * K / seconds / 1e6 (pylbm/monitoring.py:111)
-  roofline  algorithmic bytes of the fused kernel (19 loads + 19 stores of
-            4 B per cell = 152 B/cell) per launch / average launch time,
+  roofline  algorithmic bytes of a launch (19 loads + 19 stores of 4 B per cell =
+            152 B/cell, once for the steps it advances) / average launch time,
             against the 8 TB/s HBM peak; traffic = HBM bytes per launch from
             rocprofv3 FETCH_SIZE + WRITE_SIZE (profiles/), scaled by the same
             counters on a plain copy kernel of known size, or null
@@ -43,7 +43,14 @@ HBM_PEAK_GBPS = 8000.0
 BYTES = {"float32": 4, "float64": 8, "float16": 2, "bfloat16": 2}
 ERR_STEPS = 1000   # steps of the accuracy leg (the D3Q19 256^3 config states its error after 1000)
 VARIANT_WARMUP = 100   # untimed steps before each variant's 200 timed steps
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_fused_step_d3q19_256_fp32.txt")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_pair_step_d3q19_256_fp32.txt")
+
+
+def _steps_per_launch(sim):
+    """2 where run() advances two steps per launch (F and Fnew change places per launch), else 1."""
+    first = sim.container.F.ptr
+    sim.run(2)
+    return 2 if sim.container.F.ptr != first else 1
 
 
 def _time_run(sim, steps, fold=None):
@@ -424,11 +431,12 @@ def main():
         rt.free(src)
         rt.free(dst)
     sim.run(args.warmup)
+    per_launch = _steps_per_launch(sim)
     ms, wall = _time_run(sim, args.steps)
     sec = ms * 1e-3
     mlups = cells * args.steps / sec / 1e6
     alg_bytes = 2 * 19 * BYTES["float32"] * cells          # per launch
-    achieved = alg_bytes * args.steps / sec / 1e9           # GB/s
+    achieved = alg_bytes * args.steps / per_launch / sec / 1e9   # GB/s
     traffic = _traffic()
     print("bench.py: %d^3 FP32: %.4f ms per step" % (n, ms / args.steps), file=sys.stderr, flush=True)
 
@@ -458,10 +466,11 @@ def main():
             # untimed warm-up after the host-side error computation: the GPU ramps
             # back up over the first steps after an idle host pause
             v.run(VARIANT_WARMUP)
+            vper = _steps_per_launch(v)
             vms, _ = _time_run(v, 200)
             r = cells * 200 / (vms * 1e-3) / 1e6
-            vmlups[dt] = {"MLUPS": round(r, 1),
-                          "frac_of_hbm_peak": round(r * 1e6 * 2 * 19 * BYTES[dt.split("-")[0]] / 1e9
+            vmlups[dt] = {"MLUPS": round(r, 1), "steps_per_launch": vper,
+                          "frac_of_hbm_peak": round(r * 1e6 * 2 * 19 * BYTES[dt.split("-")[0]] / vper / 1e9
                                                     / HBM_PEAK_GBPS, 4)}
             del v
         sim.run(VARIANT_WARMUP, fold=False)
@@ -500,8 +509,9 @@ def main():
                    "wall_s_timed": round(wall, 4)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBPS, 4), "traffic": traffic,
-                     "kernel": "fused_step<float,true> (pull + f2m + MRT relax + m2f)",
-                     "alg_bytes_per_launch": alg_bytes},
+                     "kernel": ("pair_step<float> (two steps of pull + f2m + MRT relax + m2f)" if per_launch == 2 else
+                                "fused_step<float,true> (pull + f2m + MRT relax + m2f)"),
+                     "steps_per_launch": per_launch, "alg_bytes_per_launch": alg_bytes},
         "cpu_baseline": cpu,
     }
     out.update(extra)

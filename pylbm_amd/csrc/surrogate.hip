@@ -556,6 +556,10 @@ __global__ void __launch_bounds__(64 * FUSED_WAVES) fused_step_kernel(const E* _
 // release.  64 x 3 x (1, 2 or 4 channel quarters) workgroups; groups of the same pixels
 // lie 64 apart in the grid, on one XCD and its L2.  Two stages of four blocks are in
 // flight in registers behind the one in LDS.
+// Bound by latency: 192 or 384 workgroups, each a chain of up to 16 stages (8 x 128 x 128
+// pixels: the bytes take 4-6 us).  32 x 32 channels 18 us, 64 x 32 23 us, 32 x 64 24 us; one
+// workgroup row per tap, operands transposed on their way into LDS 16 bits at a time,
+// took 48, 90 and 83; strips of rows with all nine taps 13, 17 and 19, in another order.
 template <typename E>
 __device__ __forceinline__ typename Elem<E>::v8 read_tr(const E* base, int stride) {
   // lane (g, i): pixels 8 g + [0, 8), channel i of the 16 at base (stride elements per pixel)
