@@ -63,3 +63,20 @@ def test_pairs_equal_single_steps(hip, shape, dtype, walls, source, paired, step
         want = ref.F[k]
         assert np.array_equal(sim.F[k], want)
         assert np.array_equal(plain.F[k], want)
+
+
+def test_pairs_population_planes(hip):
+    """The other arrangement of the populations (one array each) takes the same pairs."""
+    shape = (80, 97, 160)
+    d = _flow(shape, False, False)
+    sims = [Simulation(d, dtype="float32", layout=lay) for lay in ("interleaved", "planes")]
+    rng = np.random.default_rng(4)
+    noise = 0.05 * rng.standard_normal((sims[0].ns,) + tuple(sims[0].domain.shape_halo))
+    for sim in sims:
+        for k in range(sim.ns):
+            sim.F_halo[k] = sim.F_halo[k] * (1.0 + noise[k])
+        first = sim.container.F.ptr
+        sim.run(6)
+        assert sim.container.F.ptr != first   # three launches
+    for k in range(sims[0].ns):
+        assert np.array_equal(sims[0].F[k], sims[1].F[k])
