@@ -72,9 +72,10 @@ struct f32dev {
 // Codec<S>::C is the compute type.  load/store convert a stored population
 // to/from its full value; load_dev/store_dev to/from its deviation from the
 // rest population w (= w_k rho0): the deviation formats store it directly, the
-// FP32 full-value format subtracts w (exact for w/2 <= f <= 2w).  advance: the stored
-// form of d + inc, where r is the stored form of d (decode_dev); the FP32 full-value
-// format adds inc to r itself, which rounds once.
+// FP32 full-value format subtracts w (exact for w/2 <= f <= 2w).  advance (the formats
+// with contracted collisions in deviations): the stored form of d + inc, where r is the
+// stored form of d (decode_dev); the FP32 full-value format adds inc to r itself, which
+// rounds once.
 template <typename S>
 struct Codec;
 
@@ -86,7 +87,6 @@ struct Codec<double> {
   __device__ __forceinline__ static C decode_dev(double r, C w) { return r - w; }
   __device__ __forceinline__ static double encode(C v, C) { return v; }
   __device__ __forceinline__ static double encode_dev(C d, C w) { return w + d; }
-  __device__ __forceinline__ static double advance(double, C d, C inc, C w) { return encode_dev(d + inc, w); }
   __device__ __forceinline__ static C load(const double* p, int64_t i, C) { return p[i]; }
   __device__ __forceinline__ static void store(double* p, int64_t i, C v, C) { put(p + i, v); }
   __device__ __forceinline__ static C load_dev(const double* p, int64_t i, C w) { return p[i] - w; }
@@ -118,7 +118,6 @@ struct Codec<f32dev> {
   __device__ __forceinline__ static C decode_dev(f32dev r, C) { return r.x; }
   __device__ __forceinline__ static f32dev encode(C v, C w) { return f32dev{v - w}; }
   __device__ __forceinline__ static f32dev encode_dev(C d, C) { return f32dev{d}; }
-  __device__ __forceinline__ static f32dev advance(f32dev, C d, C inc, C) { return encode_dev(d + inc, C(0)); }
   __device__ __forceinline__ static C load(const f32dev* p, int64_t i, C w) { return w + p[i].x; }
   __device__ __forceinline__ static void store(f32dev* p, int64_t i, C v, C w) { put(&p[i].x, v - w); }
   __device__ __forceinline__ static C load_dev(const f32dev* p, int64_t i, C) { return p[i].x; }

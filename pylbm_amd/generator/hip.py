@@ -651,17 +651,7 @@ fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename 
   for (int j = 0; j < VEC; ++j) {
 %(coords)s
 %(decode)s
-  if constexpr (DEV) {
-%(f2m_dev)s
-%(coll_dev)s
-%(m2f_dev)s
-%(stores_dev)s
-  } else {
-%(f2m)s
-%(coll)s
-%(m2f)s
-%(stores)s
-  }
+%(collide)s
   }
 %(vstores)s
   }
@@ -1301,17 +1291,7 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
       {
 %(tb_coords)s
 %(tb_decode)s
-      if constexpr (DEV) {
-%(tb_f2m_dev)s
-%(tb_coll_dev)s
-%(tb_m2f_dev)s
-%(tb_stores_dev)s
-      } else {
-%(tb_f2m)s
-%(tb_coll)s
-%(tb_m2f)s
-%(tb_stores)s
-      }
+%(tb_collide)s
       }
 %(tb_lds_stores)s
     }
@@ -1427,17 +1407,7 @@ __device__ __forceinline__ void pair_collide(const S (&L)[NS], S (&G)[NS],
   (void)half_dt; (void)tt; (void)cref; (void)j; (void)o; (void)m; (void)ii; (void)one_minus; (void)omega;
 %(pair_coords)s
 %(pair_decode)s
-  if constexpr (DEV) {
-%(pair_f2m_dev)s
-%(pair_coll_dev)s
-%(pair_m2f_dev)s
-%(pair_stores_dev)s
-  } else {
-%(pair_f2m)s
-%(pair_coll)s
-%(pair_m2f)s
-%(pair_stores)s
-  }
+%(pair_collide)s
 }
 
 template <typename S, bool MASK, int TY>
@@ -1697,7 +1667,7 @@ _TB_LAUNCH_NONE = r"""#define LBM_DISPATCH_BLOCKED(kind, FN, f, fn, L, p, nt, tm
 """
 
 
-def _pair_source(vel, ksym, decode, coords, f2m, f2m_dev, coll_dev, m2f_dev, stores_dev, coll, m2f, stores):
+def _pair_source(vel, ksym, decode, coords, collide):
     """The kernel that advances a 3D scheme with velocity components in {-1, 0, 1} by two
     steps per pass over memory."""
     ns = len(vel)
@@ -1753,9 +1723,7 @@ def _pair_source(vel, ksym, decode, coords, f2m, f2m_dev, coll_dev, m2f_dev, sto
                      + (" kb = opaque(kb + pop);" if k < ns - 1 else ""))
     j = "\n".join
     return (_PAIR_KERNEL % dict(
-        pair_coords=_indent(coords), pair_decode=_indent(arr(decode)), pair_f2m=_indent(f2m, 4), pair_f2m_dev=_indent(f2m_dev, 4),
-        pair_coll_dev=_indent(coll_dev, 4), pair_m2f_dev=_indent(m2f_dev, 4), pair_stores_dev=_indent(arr(stores_dev), 4),
-        pair_coll=_indent(coll, 4), pair_m2f=_indent(m2f, 4), pair_stores=_indent(arr(stores), 4),
+        pair_coords=_indent(coords), pair_decode=_indent(arr(decode)), pair_collide=_indent(arr(collide)),
         pair_lat=j(lat), pair_fetch_mask=j(fetch_mask), pair_fetch=j(fetch), pair_read1=j(read1),
         pair_write=j(write), pair_read2=j(read2), pair_store=j(store))
         ).replace("PAIR_UP", str(count["up"])).replace("PAIR_LEVEL", str(count["level"])).replace(
@@ -1897,37 +1865,49 @@ def generate_source(spec: KernelSpec) -> str:
     vstores = (["if (VEC > 1 || sizeof(I) > 4 || a.nt) {"] + ["  " + ln for ln in vstores] + ["} else {", "  const auto r_ = buffer(fn, 0);"]
                + ["  " + ln for ln in cstores] + ["}"])
 
-    # The arithmetic of the step.  With fuse (FP64, and every format in 3D) moments share
-    # partial sums and products are contracted: a quarter fewer instructions.  The
-    # FP32-compute formats of 1D and 2D schemes keep the rounding of every single product
-    # and sum: their moments are read back in FP64, where another rounding would show
-    # (6e-8) as a change of results.
+    # The arithmetic of the step.  Contracted, moments share partial sums and a product and a
+    # sum of one statement become one FMA: up to a quarter fewer instructions.  Errors
+    # against wider arithmetic, replayed on the CPU over 32 to 128 flows of 30 to 400 steps
+    # (momentum, relative to single roundings): FP64 0.83 (D3Q19), 0.96 (D2Q9); FP32 0.99 and
+    # the 2-byte formats 1.00, whose stored values round far more coarsely, with M^-1 m left
+    # out: a product there enters several populations, and fused it rounds differently in
+    # each of their sums.  FP32 deviations round every product and sum on its own: their arithmetic is
+    # what their accuracy comes from (contracted 1.07, shared sums alone 1.03; 256^3 Taylor-
+    # Green vortex after 1000 steps 4.7e-7 against 3.9e-7), and it costs them nothing
+    # (306 us per step of 256^3 in pairs either way).  The FP32-compute formats of 1D and 2D
+    # schemes do the same and keep the results they have always had bit for bit (contracted:
+    # momentum error 0.97 FP32, 0.99 deviations; 1024 x 256 channel 634 us per 200 steps
+    # instead of 670).
     fuse, fuse_dev = not rel, not rel and dim == 3
 
-    def f2m_of(on):
+    def step_lines(on, dev):
+        """f2m, collision and m2f of one cell, contracted (on) or not, in deviations (dev)
+        or full values."""
         b1 = _SumBuilder("p", on)
-        f2m_lines = _transform(b1, M, fvars, mvars, ksym, sig_f2m)
-        return ((["#pragma clang fp contract(on)"] if on else [])
-                + b1.lines + ["C %s = %s;" % (o, e) for o, e in f2m_lines])
-    f2m_block, f2m_dev_block = f2m_of(fuse), f2m_of(fuse_dev)
-    if rel:
-        coll, ma_names = _relative_collision_lines(spec)
-    else:
-        coll, ma_names = _collision_lines(spec, with_sources=True), mvars
-    b2 = _SumBuilder("r", fuse)
-    m2f_lines = _inverse_transform(b2, iM, ma_names, ["g%d" % k for k in range(ns)], ksym, sig_m2f)
-    m2f_block = b2.lines + ["const C %s = %s;" % (o, e) for o, e in m2f_lines]
-    stores = ["G%d[j] = Codec<S>::encode(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
-    if rel:
-        coll_dev, m2f_dev_block, stores_dev = coll, m2f_block, stores
-    else:
-        coll_dev, dm_names = _deviation_collision_lines(spec, fuse_dev)
-        bd = _SumBuilder("rd", fuse_dev)
-        m2f_dev_lines = _inverse_transform(bd, iM, dm_names, ["g%d" % k for k in range(ns)], ksym, sig_m2f,
-                                           tag="d")
-        m2f_dev_block = bd.lines + ["const C %s = %s;" % (o, e) for o, e in m2f_dev_lines]
-        stores_dev = [("G%d[j] = Codec<S>::advance(L%d[j], f%d, g%d, a.wshift[%d]);" % (k, k, k, k, k)) if fuse_dev else
-                      ("G%d[j] = Codec<S>::encode_dev(f%d + g%d, a.wshift[%d]);" % (k, k, k, k)) for k in range(ns)]
+        f2m = _transform(b1, M, fvars, mvars, ksym, sig_f2m)
+        out = (["#pragma clang fp contract(on)"] if on else []) + b1.lines + ["C %s = %s;" % (o, e) for o, e in f2m]
+        if rel:
+            coll, names = _relative_collision_lines(spec)
+        elif dev:
+            coll, names = _deviation_collision_lines(spec, on)
+        else:
+            coll, names = _collision_lines(spec, with_sources=True, fuse=on), mvars
+        dev = dev and not rel
+        b2 = _SumBuilder("rd" if dev else "r", on)
+        m2f = _inverse_transform(b2, iM, names, ["g%d" % k for k in range(ns)], ksym, sig_m2f, tag="d" if dev else "")
+        back = b2.lines + ["const C %s = %s;" % (o, e) for o, e in m2f]
+        if not dev:
+            back += ["G%d[j] = Codec<S>::encode(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
+        elif on:
+            back += ["G%d[j] = Codec<S>::advance(L%d[j], f%d, g%d, a.wshift[%d]);" % (k, k, k, k, k) for k in range(ns)]
+        else:
+            back += ["G%d[j] = Codec<S>::encode_dev(f%d + g%d, a.wshift[%d]);" % (k, k, k, k) for k in range(ns)]
+        return out + coll + (["{", "#pragma clang fp contract(off)"] + back + ["}"] if on and dev else back)
+    collide = (["if constexpr (DEV) {"] if not fuse_dev else ["if constexpr (Codec<S>::kind == LBM_F32D) {"])
+    collide += ["  " + ln for ln in step_lines(False, True)]
+    if fuse_dev:
+        collide += ["} else if constexpr (DEV) {"] + ["  " + ln for ln in step_lines(True, True)]
+    collide += ["} else {"] + ["  " + ln for ln in step_lines(fuse, False)] + ["}"]
 
     # ---------------------------------------------------------- f2m / m2f / eq
     b3 = _SumBuilder("p")
@@ -2132,11 +2112,7 @@ def generate_source(spec: KernelSpec) -> str:
             tb_mask=_indent(tb_mask, 8), tb_collect=_indent(tb_collect, 6), tb_entries=_indent(tb_entries), tb_apply=_indent(tb_apply, 4),
             tb_loads=_indent(tb_loads, 6), tb_sub=_indent(tb_sub, 6),
             tb_gdecl=_indent(["S %s;" % ", ".join("G%d[1]" % k for k in range(ns))], 6),
-            tb_coords=_indent(coords, 6), tb_decode=_indent(decode, 6), tb_f2m=_indent(f2m_block, 8),
-            tb_f2m_dev=_indent(f2m_dev_block, 8),
-            tb_coll_dev=_indent(coll_dev, 8), tb_m2f_dev=_indent(m2f_dev_block, 8),
-            tb_stores_dev=_indent(stores_dev, 8), tb_coll=_indent(coll, 8), tb_m2f=_indent(m2f_block, 8),
-            tb_stores=_indent(stores, 8),
+            tb_coords=_indent(coords, 6), tb_decode=_indent(decode, 6), tb_collide=_indent(collide, 6),
             tb_lds_stores=_indent(["nxt[%d * RC + lcell] = G%d[0];" % (k, k) for k in range(ns)], 6))
         tb_launch = _TB_LAUNCH % {}
     else:
@@ -2145,17 +2121,14 @@ def generate_source(spec: KernelSpec) -> str:
         # up to D3Q19: what a thread holds of more populations does not fit its registers
         if ns <= 19 and not rel and all(abs(c) <= 1 for v in vel for c in v):
             tb_launch = _PAIR_LAUNCH % {} + _TB_LAUNCH_NONE
-            tb_kernel = _pair_source(vel, ksym, decode, coords, f2m_block, f2m_dev_block, coll_dev, m2f_dev_block, stores_dev, coll,
-                                     m2f_block, stores)
+            tb_kernel = _pair_source(vel, ksym, decode, coords, collide)
     return _TEMPLATE % dict(
         tb_kernel=tb_kernel, tb_launch=tb_launch, pair_ok=int(dim == 3 and bool(tb_kernel)), unit_vel=int(all(abs(c) <= 1 for v in vel for c in v)),
         hash=spec_hash(spec), ns=ns, nc=spec.nconsm, dim=dim, paired=bool(sig_f2m),
         vel=vel_txt,
         loads=_indent(loads), bbsub=_indent(bbsub), bbsub_ok=int(ksym is not None),
         gdecl=_indent(gdecl), coords=_indent(coords, 4), decode=_indent(decode, 4), vstores=_indent(vstores),
-        f2m=_indent(f2m_block, 4), f2m_dev=_indent(f2m_dev_block, 4), coll=_indent(coll, 4), coll_dev=_indent(coll_dev, 4),
-        m2f=_indent(m2f_block, 4), m2f_dev=_indent(m2f_dev_block, 4), stores_dev=_indent(stores_dev, 4),
-        stores=_indent(stores, 4),
+        collide=_indent(collide, 2),
         f2m_loads=_indent(f2m_loads), f2m_full=_indent(f2m_full), f2m_stores=_indent(f2m_stores),
         m2f_loads=_indent(m2f_loads), m2f_full=_indent(m2f_full), m2f_stores=_indent(m2f_stores),
         eq_loads=_indent(eq_loads), eq_body=_indent(eq_body), eq_stores=_indent(eq_stores),
