@@ -288,6 +288,11 @@ typedef struct lbm_params {
   /* lbm_gen_run on the wrap path: 0 = two steps per launch where that is the faster
    * (3D), 1 = one step per launch; the same bits */
   int32_t single_steps;
+  /* lbm_gen_run and lbm_gen_run_blocked: 0 = the newest state is in d_f after an even
+   * number of steps and in d_fnew after an odd one, whatever the number of steps per
+   * launch; 1 = where the last launch leaves it, which *parity tells: an odd number of
+   * two-step launches, or of blocks, then needs no single steps or extra block */
+  int32_t launch_parity;
 } lbm_params;
 
 /* information on the generated module (ns, nconsm, dim) */
@@ -338,8 +343,9 @@ int lbm_gen_source_term(double* d_m, const lbm_layout* mlayout, const lbm_params
 /*
  * nsteps complete time steps (ghost fill, link lists in order, fused step,
  * swap) without returning to the host: pylbm/simulation.py:392-420 repeated.
- * d_f / d_fnew are swapped nsteps times; on return *parity = nsteps % 2 tells
- * which buffer holds the newest state (0: d_f).  links: nmeth descriptors.
+ * On return *parity tells which buffer holds the newest state (0: d_f): nsteps % 2,
+ * or with params->launch_parity set the number of launches, between which d_f and
+ * d_fnew change places, modulo 2.  links: nmeth descriptors.
  */
 typedef struct lbm_link_set {
   const uint32_t* d_store;

@@ -1065,7 +1065,8 @@ int lbm_gen_run_blocked(void* d_f, void* d_fnew, const lbm_layout* layout, lbm_p
   void* b = d_fnew;
   // nsteps in launches of at most steps_per_launch steps, as even as they come: 200
   // steps at most 6 at a time are 32 launches of 6 and 2 of 4, not 33 and two steps
-  const int64_t launches = (nsteps + steps_per_launch - 1) / steps_per_launch;
+  int64_t launches = (nsteps + steps_per_launch - 1) / steps_per_launch;
+  if (!params->launch_parity) launches += (nsteps - launches) & 1;
   for (int64_t it = 0; it < launches; ++it) {
     const int nt = (int)(nsteps * (it + 1) / launches - nsteps * it / launches);
     int rc = 0;
@@ -1092,10 +1093,14 @@ int lbm_gen_run(void* d_f, void* d_fnew, const lbm_layout* layout, const lbm_vel
   void* a = d_f;
   void* b = d_fnew;
   int64_t launches = 0;
+#if PAIR_OK
+  // an even number of pairs leaves the result where single steps would have
+  const int64_t paired = !periodic_fold ? 0 : params->launch_parity ? nsteps / 2 * 2 : nsteps / 4 * 4;
+#endif
   for (int64_t it = 0; it < nsteps; ++it, ++launches) {
     int rc = 0;
 #if PAIR_OK
-    if (periodic_fold && it + 2 <= nsteps) {
+    if (it < paired) {
       bool done;
       rc = pair_any(a, b, layout, params, &done, (hipStream_t)stream);
       if (rc) return rc;

@@ -54,7 +54,8 @@ class LbmParams(ctypes.Structure):
                 ("bbtab_sign", ctypes.c_void_p), ("bbtab_rhs", ctypes.c_void_p), ("bbtab_rel", ctypes.c_void_p),
                 ("bbtab_src2", ctypes.c_void_p), ("bbtab_c2", ctypes.c_void_p), ("bbtab_rel2", ctypes.c_void_p),
                 ("origin", ctypes.c_double * 3), ("dx", ctypes.c_double),
-                ("xcd_remap", ctypes.c_int32), ("vec_cells", ctypes.c_int32), ("single_steps", ctypes.c_int32)]
+                ("xcd_remap", ctypes.c_int32), ("vec_cells", ctypes.c_int32), ("single_steps", ctypes.c_int32),
+                ("launch_parity", ctypes.c_int32)]
 
 
 class LbmLinkSet(ctypes.Structure):

@@ -225,6 +225,7 @@ class Simulation:
             self.params.origin[d] = float(c[0])
         self.params.dx = float(self.domain.dx)
         self.params.xcd_remap = -1
+        self.params.launch_parity = 1   # run() exchanges F and Fnew by the parity it gets back
         vmax = list(self.domain.stencil.vmax)
         # reference state of the FP32-compute formats: conserved moments
         # (rho0, 0, ...), its equilibrium populations w_k rho0

@@ -365,10 +365,10 @@ class LatticeState:
         (several steps per launch in LDS, bit-identical to one launch per step) when
         ``blocked`` is set and the grid allows it, else one folded fused launch per
         step."""
-        if nsteps % 2 or (self.blocked and self.sim._blocking_shape() is not None):
-            self.sim.run(nsteps)
-            return
         sim = self.sim
+        if nsteps <= 0 or (self.blocked and sim._blocking_shape() is not None):
+            sim.run(nsteps)
+            return
         c = sim.container
         if getattr(self, "_bound", None) != (c.F.ptr, c.Fnew.ptr):
             self._bind()
@@ -376,6 +376,8 @@ class LatticeState:
         self.rt.check(sim.module.lbm_gen_run(ctypes.c_void_p(c.F.ptr), ctypes.c_void_p(c.Fnew.ptr), self._f_lay,
                                              self._vel, self._params, sim._link_sets, 0, int(nsteps), 0, 1,
                                              ctypes.byref(self._parity), self.rt.stream), "run")
+        if self._parity.value:
+            c.F, c.Fnew = c.Fnew, c.F
         sim._update_m = True
         sim.nt += nsteps
         sim.t = sim.t + nsteps * sim.dt

@@ -214,3 +214,31 @@ def test_overlapped_failed_judge_falls_back_to_last_passed_checkpoint(nint, je, 
         prefix = "s" * (bad * je - 1) + "L"
     assert hist == prefix + "L" * (nint - len(prefix))
     assert len(run.judges) == bad + 1
+
+
+@pytest.mark.parametrize("nsteps,parity", [(4, 0), (4, 1), (5, 1), (2, 1)])
+def test_lattice_run_exchanges_buffers_by_parity(nsteps, parity):
+    """LatticeState.run keeps the newest state in F for whatever parity the library
+    returns: with several steps per launch an even number may end in Fnew."""
+    import types
+
+    from pylbm_amd.surrogate import LatticeState
+
+    def gen_run(*args):
+        args[10]._obj.value = parity
+        return 0
+    first, second = object(), object()
+    lat = object.__new__(LatticeState)
+    lat.blocked = False
+    lat.rt = types.SimpleNamespace(check=lambda rc, what: None, stream=None)
+    lat.sim = types.SimpleNamespace(
+        container=types.SimpleNamespace(F=types.SimpleNamespace(ptr=1, array=first),
+                                        Fnew=types.SimpleNamespace(ptr=2, array=second)),
+        module=types.SimpleNamespace(lbm_gen_run=gen_run), params=types.SimpleNamespace(t=0.0), t=0.0, dt=1.0, nt=0,
+        _link_sets=None, run=lambda n: pytest.fail("not the general run"))
+    lat._bound, lat._f_lay, lat._vel, lat._params = (1, 2), None, None, None
+    lat._parity = ctypes.c_int(0)
+    lat.run(nsteps)
+    c = lat.sim.container
+    assert (c.F.array, c.Fnew.array) == ((second, first) if parity else (first, second))
+    assert lat.sim.nt == nsteps
