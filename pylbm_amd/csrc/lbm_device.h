@@ -245,18 +245,21 @@ __device__ __forceinline__ void vload_pull(S (&out)[V], const S* p) {
   }
 }
 
-template <typename S, int V>
+// with put (NT) or into the caches
+template <typename S, int V, bool NT>
 __device__ __forceinline__ void vstore(S* p, const S (&in)[V]) {
   using B = typename Bits<S>::T;
   if constexpr (V == 1) {
     B b;
     __builtin_memcpy(&b, in, sizeof(S));
-    put((B*)p, b);
+    if constexpr (NT) put((B*)p, b);
+    else *(B*)p = b;
   } else {
     typedef B vec_t __attribute__((ext_vector_type(V)));
     vec_t v;
     __builtin_memcpy(&v, in, sizeof(S) * V);
-    put((vec_t*)p, v);
+    if constexpr (NT) put((vec_t*)p, v);
+    else *(vec_t*)p = v;
   }
 }
 

@@ -616,8 +616,10 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t 
 }
 
 // I: the element index type, int32_t when every index of the array fits it (the
-// usual case: 32-bit offsets from a 64-bit base), int64_t for larger arrays
-template <typename S, bool FOLD, int VEC, typename I>
+// usual case: 32-bit offsets from a 64-bit base), int64_t for larger arrays.  NT: the
+// population stores bypass the caches (stream_stores); a branch on it inside the kernel
+// would be merged into one kind of store.
+template <typename S, bool FOLD, int VEC, typename I, bool NT>
 __global__ void __launch_bounds__(LBM_BX * block_rows<S>())
 fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Codec<S>::C> a) {
   using C = typename Codec<S>::C;
@@ -792,6 +794,7 @@ eq_m2f_kernel(const double* __restrict__ mo, lbm_layout ml, S* __restrict__ f, l
 // into the caches: 64^3 FP32 10.2 / 8.7, FP64 18.1 / 14.7, 96^3 FP32 26.2 / 23.4, 128^3 FP32
 // (319 MB) 59 / 54; 128^3 FP64 (637 MB) 113 / 125, 160^3 FP32 106 / 118).  Small grids wait
 // for the L2s to be written back at the end of every step (64^2 FP64 4.7 / 5.6).
+// Launches of four cells per thread and 64-bit indices always bypass them.
 static int stream_stores(const lbm_layout* L) {
   const int64_t bytes = 2 * L->n[0] * L->n[1] * L->pitch * L->ns * (int64_t)storage_elem_size(L->storage);
   return bytes < (int64_t)24 << 20 || bytes > (int64_t)320 << 20;
@@ -845,6 +848,22 @@ static unsigned block_x(int64_t n) {
   return n >= 256 ? 256u : (n >= 128 ? 128u : 64u);
 }
 
+template <typename S, bool FOLD>
+static void fused_launch(const S* f, S* fn, const StepArgs<typename Codec<S>::C>& a, bool narrow, int vec, dim3 grid,
+                         dim3 block, hipStream_t s) {
+  constexpr int V = vec_cells<S>();
+  const auto go = [&](auto kernel) { kernel<<<grid, block, 0, s>>>(f, fn, a); };
+  if (vec == V && V > 1) {
+    if (narrow) go(fused_step<S, FOLD, V, int32_t, true>);
+    else go(fused_step<S, FOLD, V, int64_t, true>);
+  } else if (!narrow) {
+    go(fused_step<S, FOLD, 1, int64_t, true>);
+  } else {
+    if (a.nt) go(fused_step<S, FOLD, 1, int32_t, true>);
+    else go(fused_step<S, FOLD, 1, int32_t, false>);
+  }
+}
+
 template <typename S>
 static int step_launch(const void* f, void* fn, const lbm_layout* L, const lbm_params* p, int fold,
                        hipStream_t s) {
@@ -880,23 +899,9 @@ static int step_launch(const void* f, void* fn, const lbm_layout* L, const lbm_p
     for (int d = 0; d < 3; ++d)
       LBM_REQUIRE(a.nin[d] >= a.halo[d], "periodic fold needs extents >= halo");
   }
-  if (layout_fits_int32(*L) && !LBM_FORCE_I64) {
-    if (vec == V) {
-      if (fold) fused_step<S, true, V, int32_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-      else fused_step<S, false, V, int32_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-    } else {
-      if (fold) fused_step<S, true, 1, int32_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-      else fused_step<S, false, 1, int32_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-    }
-  } else {
-    if (vec == V) {
-      if (fold) fused_step<S, true, V, int64_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-      else fused_step<S, false, V, int64_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-    } else {
-      if (fold) fused_step<S, true, 1, int64_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-      else fused_step<S, false, 1, int64_t><<<grid, block, 0, s>>>((const S*)f, (S*)fn, a);
-    }
-  }
+  const bool narrow = layout_fits_int32(*L) && !LBM_FORCE_I64;
+  if (fold) fused_launch<S, true>((const S*)f, (S*)fn, a, narrow, vec, grid, block, s);
+  else fused_launch<S, false>((const S*)f, (S*)fn, a, narrow, vec, grid, block, s);
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1864,11 +1869,7 @@ def generate_source(spec: KernelSpec) -> str:
     else:
         decode = ["C f%d = DEV ? Codec<S>::decode_dev(L%d[j], a.wshift[%d]) : Codec<S>::decode(L%d[j], a.wshift[%d]);"
                   % (k, k, k, k, k) for k in range(ns)]
-    vstores = ["vstore<S, VEC>(fn + ((I)a.dst_off[%d] + cell), G%d);" % (k, k) for k in range(ns)]
-    cstores = ["buffer_store<S, false>(r_, (uint32_t)(cell * sizeof(S)), (uint32_t)(a.dst_off[%d] * sizeof(S)), G%d[0]);"
-               % (k, k) for k in range(ns)]
-    vstores = (["if (VEC > 1 || sizeof(I) > 4 || a.nt) {"] + ["  " + ln for ln in vstores] + ["} else {", "  const auto r_ = buffer(fn, 0);"]
-               + ["  " + ln for ln in cstores] + ["}"])
+    vstores = ["vstore<S, VEC, NT>(fn + ((I)a.dst_off[%d] + cell), G%d);" % (k, k) for k in range(ns)]
 
     # The arithmetic of the step.  Contracted, moments share partial sums and a product and a
     # sum of one statement become one FMA: up to a quarter fewer instructions.  Errors

@@ -52,3 +52,13 @@ def test_printed_transforms_are_exact():
     env2 = _eval_block(kern[start:], kern[start:start + 10], "G0[j] = Codec<S>::encode(", env2)
     g = np.array([env2["g%d" % k] for k in range(spec.ns)])
     assert np.allclose(g, iM @ m2, rtol=1e-13, atol=1e-14)
+
+
+def test_fused_step_addresses_stores_by_element_index():
+    """The step's stores take the index type of the launch: 32-bit byte offsets would wrap
+    in a layout whose strides span 4 GiB with fewer than 2^31 elements."""
+    src = generate_source(Scheme(cases.taylor_green_d3q19(4)).kernel_spec())
+    kern = src[src.index("fused_step(const S*"):]
+    kern = kern[:kern.index("\n}\n")]
+    assert kern.count("fn + ((I)a.dst_off[") == 19
+    assert "buffer_store" not in kern and "uint32_t)(cell" not in kern
