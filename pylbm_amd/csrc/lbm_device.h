@@ -72,10 +72,7 @@ struct f32dev {
 // Codec<S>::C is the compute type.  load/store convert a stored population
 // to/from its full value; load_dev/store_dev to/from its deviation from the
 // rest population w (= w_k rho0): the deviation formats store it directly, the
-// FP32 full-value format subtracts w (exact for w/2 <= f <= 2w).  advance (the formats
-// with contracted collisions in deviations): the stored form of d + inc, where r is the
-// stored form of d (decode_dev); the FP32 full-value format adds inc to r itself, which
-// rounds once.
+// FP32 full-value format subtracts / adds w (exact for w/2 <= f <= 2w).
 template <typename S>
 struct Codec;
 
@@ -102,7 +99,6 @@ struct Codec<float> {
   __device__ __forceinline__ static C decode_dev(float r, C w) { return r - w; }
   __device__ __forceinline__ static float encode(C v, C) { return v; }
   __device__ __forceinline__ static float encode_dev(C d, C w) { return w + d; }
-  __device__ __forceinline__ static float advance(float r, C, C inc, C) { return r + inc; }
   __device__ __forceinline__ static C load(const float* p, int64_t i, C) { return p[i]; }
   __device__ __forceinline__ static void store(float* p, int64_t i, C v, C) { put(p + i, v); }
   __device__ __forceinline__ static C load_dev(const float* p, int64_t i, C w) { return p[i] - w; }
@@ -133,7 +129,6 @@ struct Codec<_Float16> {
   __device__ __forceinline__ static C decode_dev(_Float16 r, C) { return (float)r; }
   __device__ __forceinline__ static _Float16 encode(C v, C w) { return (_Float16)(v - w); }
   __device__ __forceinline__ static _Float16 encode_dev(C d, C) { return (_Float16)d; }
-  __device__ __forceinline__ static _Float16 advance(_Float16, C d, C inc, C) { return encode_dev(d + inc, C(0)); }
   __device__ __forceinline__ static C load(const _Float16* p, int64_t i, C w) {
     return w + (float)p[i];
   }
@@ -153,7 +148,6 @@ struct Codec<bf16> {
   __device__ __forceinline__ static C decode_dev(bf16 r, C) { return bf16_to_float(r); }
   __device__ __forceinline__ static bf16 encode(C v, C w) { return float_to_bf16(v - w); }
   __device__ __forceinline__ static bf16 encode_dev(C d, C) { return float_to_bf16(d); }
-  __device__ __forceinline__ static bf16 advance(bf16, C d, C inc, C) { return encode_dev(d + inc, C(0)); }
   __device__ __forceinline__ static C load(const bf16* p, int64_t i, C w) {
     return w + bf16_to_float(p[i]);
   }

@@ -1872,19 +1872,18 @@ def generate_source(spec: KernelSpec) -> str:
     vstores = ["vstore<S, VEC, NT>(fn + ((I)a.dst_off[%d] + cell), G%d);" % (k, k) for k in range(ns)]
 
     # The arithmetic of the step.  Contracted, moments share partial sums and a product and a
-    # sum of one statement become one FMA: up to a quarter fewer instructions.  Errors
-    # against wider arithmetic, replayed on the CPU over 32 to 128 flows of 30 to 400 steps
-    # (momentum, relative to single roundings): FP64 0.83 (D3Q19), 0.96 (D2Q9); FP32 0.99 and
-    # the 2-byte formats 1.00, whose stored values round far more coarsely, with M^-1 m left
-    # out: a product there enters several populations, and fused it rounds differently in
-    # each of their sums.  FP32 deviations round every product and sum on its own: their arithmetic is
-    # what their accuracy comes from (contracted 1.07, shared sums alone 1.03; 256^3 Taylor-
-    # Green vortex after 1000 steps 4.7e-7 against 3.9e-7), and it costs them nothing
-    # (306 us per step of 256^3 in pairs either way).  The FP32-compute formats of 1D and 2D
-    # schemes do the same and keep the results they have always had bit for bit (contracted:
-    # momentum error 0.97 FP32, 0.99 deviations; 1024 x 256 channel 634 us per 200 steps
-    # instead of 670).
-    fuse, fuse_dev = not rel, not rel and dim == 3
+    # sum of one statement become one FMA: up to a quarter fewer instructions.  FP64 does
+    # (errors against wider arithmetic, replayed on the CPU over 32 flows of 30 to 400 steps,
+    # relative to single roundings: momentum 0.83 in D3Q19, 0.96 in D2Q9; 128^3 in pairs 84 ->
+    # 78 us per step), and so do the 2-byte formats in 3D, whose stored values round 2^13
+    # times more coarsely (momentum 1.00 over 128 flows; 128^3 27.0 -> 25.2 us), but for M^-1 m:
+    # a product there enters several populations, and fused it rounds differently in each of their sums.
+    # FP32 and its deviations round every product and sum on its own: deviations get their
+    # accuracy from their arithmetic (contracted 1.07, shared sums alone 1.03; 256^3 Taylor-
+    # Green vortex after 1000 steps 4.7e-7 against 3.9e-7, 306 us per step either way), and FP32
+    # gains 1 to 3 % in pairs (256^3 308 -> 305 us) and loses as much in single steps of large
+    # boxes (230 x 210 x 220 308 -> 317 us).
+    fuse, fuse_16 = not rel, not rel and dim == 3
 
     def step_lines(on, dev):
         """f2m, collision and m2f of one cell, contracted (on) or not, in deviations (dev)
@@ -1902,16 +1901,14 @@ def generate_source(spec: KernelSpec) -> str:
         b2 = _SumBuilder("rd" if dev else "r", on)
         m2f = _inverse_transform(b2, iM, names, ["g%d" % k for k in range(ns)], ksym, sig_m2f, tag="d" if dev else "")
         back = b2.lines + ["const C %s = %s;" % (o, e) for o, e in m2f]
-        if not dev:
-            back += ["G%d[j] = Codec<S>::encode(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
-        elif on:
-            back += ["G%d[j] = Codec<S>::advance(L%d[j], f%d, g%d, a.wshift[%d]);" % (k, k, k, k, k) for k in range(ns)]
-        else:
+        if dev:
             back += ["G%d[j] = Codec<S>::encode_dev(f%d + g%d, a.wshift[%d]);" % (k, k, k, k) for k in range(ns)]
+        else:
+            back += ["G%d[j] = Codec<S>::encode(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
         return out + coll + (["{", "#pragma clang fp contract(off)"] + back + ["}"] if on and dev else back)
-    collide = (["if constexpr (DEV) {"] if not fuse_dev else ["if constexpr (Codec<S>::kind == LBM_F32D) {"])
+    collide = ["if constexpr (%s) {" % ("DEV && sizeof(S) > 2" if fuse_16 else "DEV")]
     collide += ["  " + ln for ln in step_lines(False, True)]
-    if fuse_dev:
+    if fuse_16:
         collide += ["} else if constexpr (DEV) {"] + ["  " + ln for ln in step_lines(True, True)]
     collide += ["} else {"] + ["  " + ln for ln in step_lines(fuse, False)] + ["}"]
 
