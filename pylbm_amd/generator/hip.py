@@ -565,6 +565,20 @@ __host__ __device__ constexpr int block_rows() {
   return LBM_BY > 1 ? LBM_BY : (sizeof(S) == 8 ? 2 : 1);
 }
 
+// Waves per SIMD of a fused step.  FP64 in 3D, at least 4: source terms in X, Y, Z and t
+// bring D3Q19 to 129 registers, one more than 4 waves have (200^3 431 us per step with 3).
+// 2-byte formats in 3D with stores past the caches, at most 5: with 6, 200^3 FP16 takes 135
+// us instead of 129, 230 x 210 x 220 164 instead of 158; 16 populations and more (6
+// populations stream faster with all 8, 200^3 47 us instead of 58).
+template <typename S, bool TABLE>
+constexpr int least_waves() {
+  return sizeof(S) == 8 && DIM == 3 && NS <= 19 && !TABLE ? 4 : 1;
+}
+template <typename S, bool NT>
+constexpr int most_waves() {
+  return sizeof(S) == 2 && DIM == 3 && NS >= 16 && NT ? 5 : 8;
+}
+
 template <typename S>
 constexpr int vec_cells() {
   return LBM_VEC > 0 ? LBM_VEC : (sizeof(S) <= 4 ? 4 : 1);
@@ -618,9 +632,11 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t 
 // I: the element index type, int32_t when every index of the array fits it (the
 // usual case: 32-bit offsets from a 64-bit base), int64_t for larger arrays.  NT: the
 // population stores bypass the caches (stream_stores); a branch on it inside the kernel
-// would be merged into one kind of store.
-template <typename S, bool FOLD, int VEC, typename I, bool NT>
+// would be merged into one kind of store.  TABLE: folded links may have table entries; their
+// batched loads take registers (D2Q9 FP64 48 -> 130) that boxes without a table need not pay.
+template <typename S, bool FOLD, int VEC, typename I, bool NT, bool TABLE>
 __global__ void __launch_bounds__(LBM_BX * block_rows<S>())
+__attribute__((amdgpu_waves_per_eu(least_waves<S, TABLE>(), most_waves<S, NT>())))
 fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Codec<S>::C> a) {
   using C = typename Codec<S>::C;
   // full-value arithmetic for FP64 (as pylbm), deviations from the rest state otherwise
@@ -631,7 +647,7 @@ fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename 
   if (i >= a.nin[2]) return;
   // with table entries the planes go from both ends to the middle: inflow and outflow faces,
   // whose waves take several times as long, do not come last
-  const int oo = a.ends_first ? ((bkz & 1) ? a.nin[0] - 1 - (int)(bkz >> 1) : (int)(bkz >> 1)) : (int)bkz;
+  const int oo = TABLE && a.ends_first ? ((bkz & 1) ? a.nin[0] - 1 - (int)(bkz >> 1) : (int)(bkz >> 1)) : (int)bkz;
   const int mbase = (bky * blockDim.y + threadIdx.y) * LBM_MROWS;
   const C half_dt = a.half_dt;
   const C tt = a.t;
@@ -848,20 +864,21 @@ static unsigned block_x(int64_t n) {
   return n >= 256 ? 256u : (n >= 128 ? 128u : 64u);
 }
 
-template <typename S, bool FOLD>
+template <typename S, bool FOLD, bool TABLE>
 static void fused_launch(const S* f, S* fn, const StepArgs<typename Codec<S>::C>& a, bool narrow, int vec, dim3 grid,
                          dim3 block, hipStream_t s) {
   constexpr int V = vec_cells<S>();
   const auto go = [&](auto kernel) { kernel<<<grid, block, 0, s>>>(f, fn, a); };
-  if (vec == V && V > 1) {
-    if (narrow) go(fused_step<S, FOLD, V, int32_t, true>);
-    else go(fused_step<S, FOLD, V, int64_t, true>);
-  } else if (!narrow) {
-    go(fused_step<S, FOLD, 1, int64_t, true>);
-  } else {
-    if (a.nt) go(fused_step<S, FOLD, 1, int32_t, true>);
-    else go(fused_step<S, FOLD, 1, int32_t, false>);
+  if constexpr (V > 1 && !TABLE) {
+    if (vec == V) {
+      if (narrow) go(fused_step<S, FOLD, V, int32_t, true, false>);
+      else go(fused_step<S, FOLD, V, int64_t, true, false>);
+      return;
+    }
   }
+  if (!narrow) go(fused_step<S, FOLD, 1, int64_t, true, TABLE>);
+  else if (a.nt) go(fused_step<S, FOLD, 1, int32_t, true, TABLE>);
+  else go(fused_step<S, FOLD, 1, int32_t, false, TABLE>);
 }
 
 template <typename S>
@@ -885,7 +902,8 @@ static int step_launch(const void* f, void* fn, const lbm_layout* L, const lbm_p
   LBM_REQUIRE(want == 0 || want == 1 || (want == V && a.nin[2] %% V == 0),
               "vec_cells %%d not available (%%d cells per thread, contiguous extent %%d)", want, V, a.nin[2]);
   const bool auto_vec = (sizeof(S) != 2 || LBM_VEC16_AUTO) && fold && a.bbmask == nullptr;
-  const int vec = want ? want : ((auto_vec && a.nin[2] %% V == 0 && cells / V >= ((int64_t)1 << 20)) ? V : 1);
+  // cells with table entries are updated one per thread
+  const int vec = a.bbtab_bits ? 1 : want ? want : ((auto_vec && a.nin[2] %% V == 0 && cells / V >= ((int64_t)1 << 20)) ? V : 1);
   a.remap = (p && p->xcd_remap >= 0) ? (p->xcd_remap != 0) : !fold;
   a.ends_first = fold && a.bbtab_bits && !a.remap;
   const int threads = a.nin[2] / vec;
@@ -900,8 +918,12 @@ static int step_launch(const void* f, void* fn, const lbm_layout* L, const lbm_p
       LBM_REQUIRE(a.nin[d] >= a.halo[d], "periodic fold needs extents >= halo");
   }
   const bool narrow = layout_fits_int32(*L) && !LBM_FORCE_I64;
-  if (fold) fused_launch<S, true>((const S*)f, (S*)fn, a, narrow, vec, grid, block, s);
-  else fused_launch<S, false>((const S*)f, (S*)fn, a, narrow, vec, grid, block, s);
+  const auto go = [&](auto folded, auto table) {
+    fused_launch<S, decltype(folded)::value, decltype(table)::value>((const S*)f, (S*)fn, a, narrow, vec, grid, block, s);
+  };
+  using T = std::integral_constant<bool, BBSUB_OK>;
+  if (fold) a.bbtab_bits ? go(std::true_type{}, T{}) : go(std::true_type{}, std::false_type{});
+  else a.bbtab_bits ? go(std::false_type{}, T{}) : go(std::false_type{}, std::false_type{});
   LBM_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1780,16 +1802,17 @@ def generate_source(spec: KernelSpec) -> str:
                  "#pragma unroll",
                  "    for (int j = 0; j < VEC; ++j) {",
                  "      const uint32_t bits = a.bbmask[mc + j];",
-                 "      if (bits) {",
-                 "        uint32_t tb = 0, tbase = 0;",
-                 "        if (bits & 0x80000000u) {",
-                 "          tb = a.bbtab_bits[mc + j];",
-                 "          tbase = a.bbtab_base[mc + j];",
-                 "        }",
-                 "        (void)tbase;"]
+                 "      if (bits) {"]
         for k in range(ns):
             if ksym[k] != k:
                 bbsub.append("        if (bits & %du) L%d[j] = f[(I)a.dst_off[%d] + cell + j];" % (1 << k, k, ksym[k]))
+        bbsub += ["        if constexpr (TABLE) {",
+                  "        uint32_t tb = 0, tbase = 0;",
+                  "        if (bits & 0x80000000u) {",
+                  "          tb = a.bbtab_bits[mc + j];",
+                  "          tbase = a.bbtab_base[mc + j];",
+                  "        }",
+                  "        (void)tbase;"]
         # directions that leave through the same face together: its cells need one or two
         linked = sorted((k for k in range(ns) if ksym[k] != k), key=lambda k: vel[k])
         size = 8 if ns <= 9 else 3
@@ -1824,7 +1847,7 @@ def generate_source(spec: KernelSpec) -> str:
                           "              L%d[j] = Codec<S>::encode(r_, (CC)0);" % k,
                           "            }"]
             bbsub += ["          }", "        }"]
-        bbsub += ["      }", "    }", "  }", "}"]
+        bbsub += ["        }", "      }", "    }", "  }", "}"]
     loads = ["S %s;" % ", ".join("L%d[VEC]" % k for k in range(ns))]
     loads.append("if (!FOLD) {")
     for k in range(ns):

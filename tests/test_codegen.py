@@ -62,3 +62,30 @@ def test_fused_step_addresses_stores_by_element_index():
     kern = kern[:kern.index("\n}\n")]
     assert kern.count("fn + ((I)a.dst_off[") == 19
     assert "buffer_store" not in kern and "uint32_t)(cell" not in kern
+
+
+def test_step_without_a_table_keeps_its_registers(tmp_path):
+    """The loads of table entries stay out of the kernels that boxes without a table run: the
+    D3Q6 FP64 step fits the 64 registers of 8 waves per SIMD (compiled here, not run)."""
+    import os
+    import subprocess
+    from pylbm_amd import demos
+    from pylbm_amd.generator.build import CSRC, HIPCC, HIPCC_FLAGS, INCLUDE
+    src = tmp_path / "d3q6.hip"
+    src.write_text(generate_source(Scheme(demos.advection_3d(1 / 8)[0]).kernel_spec()))
+    flags = [f for f in HIPCC_FLAGS if f != "-shared"]
+    out = subprocess.run([HIPCC] + flags + ["-I" + INCLUDE, "-I" + CSRC, "--cuda-device-only", "-c", str(src), "-o",
+                                            os.devnull, "-Rpass-analysis=kernel-resource-usage"],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, check=True).stdout
+    vgprs = {}
+    for line in out.splitlines():
+        name = re.search(r"Function Name: (\S+)", line)
+        if name:
+            kernel = name.group(1)
+        count = re.search(r"    VGPRs: (\d+)", line)
+        if count:
+            vgprs[kernel] = int(count.group(1))
+    steps = {k: v for k, v in vgprs.items() if "fused_stepId" in k}   # FP64
+    assert len(steps) >= 6 and min(steps.values()) <= 64
+    wrap = [v for k, v in steps.items() if "fused_stepIdLb1E" in k]   # periodic fold
+    assert sum(v <= 64 for v in wrap) >= len(wrap) // 2, steps
