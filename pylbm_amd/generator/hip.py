@@ -805,15 +805,20 @@ eq_m2f_kernel(const double* __restrict__ mo, lbm_layout ml, S* __restrict__ f, l
 %(m2f_stores)s
 }
 
-// Population stores bypass the caches, unless both arrays together are 24 to 320 MB: the
-// next step then finds them in the 256 MB Infinity Cache (us per step of D3Q19, past /
-// into the caches: 64^3 FP32 10.2 / 8.7, FP64 18.1 / 14.7, 96^3 FP32 26.2 / 23.4, 128^3 FP32
-// (319 MB) 59 / 54; 128^3 FP64 (637 MB) 113 / 125, 160^3 FP32 106 / 118).  Small grids wait
-// for the L2s to be written back at the end of every step (64^2 FP64 4.7 / 5.6).
-// Launches of four cells per thread and 64-bit indices always bypass them.
-static int stream_stores(const lbm_layout* L) {
-  const int64_t bytes = 2 * L->n[0] * L->n[1] * L->pitch * L->ns * (int64_t)storage_elem_size(L->storage);
-  return bytes < (int64_t)24 << 20 || bytes > (int64_t)320 << 20;
+// Population stores bypass the caches, unless the interior cells of both arrays hold 24 MiB
+// to a limit: the next step then finds them in the 256 MB Infinity Cache.  The padding of the
+// rows is not stored, so it does not count.  us per step past / into the caches:
+// below 24 MiB: 64^3 D3Q19 FP16 (19 MiB) 7.1 / 7.8, 40^3 FP64 (19) 7.6 / 8.1, 512^2 D2Q9 FP32
+// (18) 6.4 / 6.7; above: 56^3 FP32 (25) 8.3 / 8.1, 72^3 FP16 (27) 11.5 / 10.6, 96^3 FP32 (128) 26.1 / 23.0.
+// Single steps to 306 MiB: 96^3 FP64 (257) 49.1 / 45.4, 128^3 FP32 (304) 61.0 / 53.4, 136^3
+// FP32 (365) 75 / 105, 112^3 FP64 (407) 75.9 / 83.4.  2-byte formats in 3D to 176 MiB: 128^3 FP16
+// (152) 29.2 / 25.4, D3Q15 160^3 (235) 47 / 51, 160^3 (297) 61 / 68.  Pairs to 256 MiB: 112^3 FP32
+// (204) 38.0 / 32.6, 120^3 FP32 (251) 43.2 / 40.3, 96^3 FP64 (257) 35.3 / 37.0, D3Q6 180^3 FP32
+// (267) 38.5 / 40.4.
+static int stream_stores(const lbm_layout* L, int64_t most) {
+  int64_t bytes = 2 * (int64_t)L->ns * storage_elem_size(L->storage);
+  for (int d = 0; d < 3; ++d) bytes *= L->n[d] - 2 * L->halo[d];
+  return bytes < (int64_t)24 << 20 || bytes > most << 20;
 }
 
 template <typename C>
@@ -835,7 +840,7 @@ static int make_args(const lbm_layout* L, const lbm_params* p, StepArgs<C>* a) {
   a->lead = (int32_t)L->lead;
   a->remap = 0;
   a->ends_first = 0;
-  a->nt = stream_stores(L);
+  a->nt = stream_stores(L, storage_elem_size(L->storage) == 2 && DIM == 3 ? 176 : 306);
   for (int k = 0; k < NS; ++k) {
     a->omega[k] = p ? (C)p->omega[k] : (C)0;
     a->one_minus[k] = p ? (C)p->one_minus[k] : (C)1;
@@ -901,7 +906,9 @@ static int step_launch(const void* f, void* fn, const lbm_layout* L, const lbm_p
   const int want = p ? p->vec_cells : 0;
   LBM_REQUIRE(want == 0 || want == 1 || (want == V && a.nin[2] %% V == 0),
               "vec_cells %%d not available (%%d cells per thread, contiguous extent %%d)", want, V, a.nin[2]);
-  const bool auto_vec = (sizeof(S) != 2 || LBM_VEC16_AUTO) && fold && a.bbmask == nullptr;
+  // Stores into the caches go one cell per thread (180^3 D3Q6 FP32 46 us per step, 53 with 4
+  // past them).
+  const bool auto_vec = (sizeof(S) != 2 || LBM_VEC16_AUTO) && fold && a.bbmask == nullptr && a.nt;
   // cells with table entries are updated one per thread
   const int vec = a.bbtab_bits ? 1 : want ? want : ((auto_vec && a.nin[2] %% V == 0 && cells / V >= ((int64_t)1 << 20)) ? V : 1);
   a.remap = (p && p->xcd_remap >= 0) ? (p->xcd_remap != 0) : !fold;
@@ -1554,6 +1561,7 @@ static int pair_launch(const void* f, void* fn, const lbm_layout* L, lbm_params*
   t.tiles_m = (a.nin[1] + TY - 1) / TY;
   t.ty = (a.nin[1] + t.tiles_m - 1) / t.tiles_m;
   t.nz = nz;
+  a.nt = stream_stores(L, 256);
   for (int q = 0; q < 2; ++q) {
     t.times[q] = (C)p->t;
     p->t += p->dt;

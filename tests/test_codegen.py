@@ -89,3 +89,30 @@ def test_step_without_a_table_keeps_its_registers(tmp_path):
     assert len(steps) >= 6 and min(steps.values()) <= 64
     wrap = [v for k, v in steps.items() if "fused_stepIdLb1E" in k]   # periodic fold
     assert sum(v <= 64 for v in wrap) >= len(wrap) // 2, steps
+
+
+def test_rule_of_the_cached_stores(tmp_path):
+    """The rule counts what a step stores, not the padding of the rows: 64^3 FP16 (19 MiB in
+    rows padded to three times that) bypasses the caches, 128^3 FP32 (304 MiB) does not."""
+    import ctypes
+    import os
+    import subprocess
+    from pylbm_amd.generator.build import INCLUDE
+    from pylbm_amd.runtime import LBM_F16D, LBM_F32, LBM_F64
+    from pylbm_amd.storage import make_layout
+    src = generate_source(Scheme(cases.taylor_green_d3q19(4)).kernel_spec())
+    fn = src[src.index("static int stream_stores("):]
+    fn = fn[:fn.index("\n}\n") + 3].replace("static int", 'extern "C" int', 1)
+    cpp, so = tmp_path / "rule.cpp", str(tmp_path / "rule.so")
+    cpp.write_text('#include "pylbm_hip.h"\nstatic int storage_elem_size(int s) { return s == %d ? 2 : s == %d ? 4 : 8; }\n'
+                   % (LBM_F16D, LBM_F32) + fn)
+    subprocess.run(["g++", "-shared", "-fPIC", "-I" + INCLUDE, str(cpp), "-o", so], check=True)
+    rule = ctypes.CDLL(os.path.abspath(so)).stream_stores
+    rule.argtypes = [ctypes.c_void_p, ctypes.c_int64]
+    for n, storage, most, past in ((64, LBM_F16D, 176, 1), (72, LBM_F16D, 176, 0), (128, LBM_F16D, 176, 0),
+                                   (160, LBM_F16D, 176, 1), (48, LBM_F32, 306, 1), (56, LBM_F32, 306, 0),
+                                   (128, LBM_F32, 306, 0), (136, LBM_F32, 306, 1), (96, LBM_F64, 306, 0),
+                                   (96, LBM_F64, 256, 1), (120, LBM_F32, 256, 0), (1024, LBM_F64, 306, 1)):
+        for interleaved in (False, True):
+            L = make_layout(19, (n + 2,) * 3, (1, 1, 1), storage, interleaved)
+            assert rule(ctypes.byref(L), most) == past, (n, storage, most)
