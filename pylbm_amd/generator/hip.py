@@ -1611,6 +1611,20 @@ static int pair_planes(const int32_t (&nin)[3]) {
   return planes;
 }
 
+// whether the compiler spilled registers of the kernel to scratch memory: a reload there waits
+// for every load in flight, and single steps are faster (D3Q19 FP64 with a source term of sines
+// of X, Y, Z and t, 10 registers spilled: 200^3 421 us per step one at a time, 468 in pairs; a
+// source linear in X, Y and Z fits: 424 and 354; 96^3 with few workgroups 51 and 51)
+template <typename S, bool MASK>
+static bool pair_spills() {
+  static const bool spills = [] {
+    hipFuncAttributes at;
+    const hipError_t e = hipFuncGetAttributes(&at, (const void*)pair_step<S, MASK, pair_rows<S, MASK>()>);
+    return e != hipSuccess || at.localSizeBytes > 0;
+  }();
+  return spills;
+}
+
 // one launch of the two-step kernel, where it is the faster one (*done)
 template <typename S, bool MASK>
 static int pair_try(const void* f, void* fn, const lbm_layout* L, lbm_params* p, bool* done, hipStream_t s) {
@@ -1620,7 +1634,7 @@ static int pair_try(const void* f, void* fn, const lbm_layout* L, lbm_params* p,
   for (int d = 0; d < 3; ++d) nin[d] = (int32_t)(L->n[d] - 2 * L->halo[d]);
   if (pair_lds<S, pair_rows<S, MASK>()>() > 160 * 1024 || reach >= ((int64_t)1 << 32) - (1 << 20) || nin[0] < 4 || nin[1] < 32 || nin[2] < 32) return 0;
   const int nz = pair_planes<S, MASK>(nin);
-  if (nz == 0) return 0;
+  if (nz == 0 || pair_spills<S, MASK>()) return 0;
   *done = true;
   return pair_launch<S, MASK>(f, fn, L, p, nz, s);
 }
