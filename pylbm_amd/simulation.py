@@ -225,6 +225,8 @@ class Simulation:
             self.params.origin[d] = float(c[0])
         self.params.dx = float(self.domain.dx)
         self.params.xcd_remap = -1
+        # asked by every run(): not worth 5 us each time
+        self._unit_velocities = bool(np.all(np.abs(np.asarray(self.scheme.stencil.get_all_velocities())) <= 1))
         self.params.launch_parity = 1   # run() exchanges F and Fnew by the parity it gets back
         vmax = list(self.domain.stencil.vmax)
         # reference state of the FP32-compute formats: conserved moments
@@ -800,8 +802,8 @@ class Simulation:
         c = self.container
         self.params.t = self.t
         parity = ctypes.c_int(0)
-        tb = self._blocking_shape() if fold else None
-        if tb is not None and nsteps > 1:
+        tb = self._blocking_shape() if fold and nsteps > 1 else None
+        if tb is not None:
             nt, tm, ti = tb
             self._check(self.module.lbm_gen_run_blocked(ctypes.c_void_p(c.F.ptr), ctypes.c_void_p(c.Fnew.ptr),
                                                         ctypes.byref(c.F.layout), ctypes.byref(self.params),
@@ -830,9 +832,7 @@ class Simulation:
         None: 1D and 2D schemes on the wrap path (periodic, or every list folded with
         its table sources within one cell) with velocity components in {-1, 0, 1}.
         The tile and its halo live in LDS (_blocked_tile)."""
-        if not self.temporal_blocking or self.dim > 2 or not self._wrap:
-            return None
-        if np.any(np.abs(np.asarray(self.scheme.stencil.get_all_velocities())) > 1):
+        if not self.temporal_blocking or self.dim > 2 or not self._wrap or not self._unit_velocities:
             return None
         if (self.params.bbtab_bits and not self.params.bbtab_rel) or (self.params.bbtab_src2 and
                                                                       not self.params.bbtab_rel2):
