@@ -56,57 +56,83 @@ FOLD_TABLE_MAX = 1 << 16
 # and 0.77 us this way.
 TB_SHAPE_1D = (64, 128)
 TB_PLANE_1D = 256
+# Steps of a run from which on the evenness of its launches no longer matters to their number
+LONG_RUN = 32
 
 
 @functools.lru_cache(maxsize=256)
-def _blocked_tile(ns, es, n0, n1, links):
-    """(steps per launch, tile rows, tile columns) of the temporally blocked 2D run of a
-    scheme of ns populations of es bytes on n0 x n1 cells, with folded links or
-    without; None when no tile fits the LDS or one launch per step is as fast.
+def _blocked_tile(ns, es, n0, n1, links, nsteps):
+    """(steps per launch, tile rows, tile columns) of a temporally blocked 2D run of nsteps
+    steps of a scheme of ns populations of es bytes on n0 x n1 cells, with folded links
+    or without; None when no tile fits the LDS or one launch per step is as fast.
 
     A workgroup keeps two copies of its tile and a halo of steps cells in LDS: many
     steps per launch share the launch and the load but recompute the halo, small tiles
     fill the GPU but have more halo, two workgroups share a CU when a region fits half
     its LDS.  The tile is the one whose estimated time per step is the least of
-    steps 2-12 x rows 4-48 x columns 8-64.  The estimate (us per launch; a sweep of
-    those tiles on MI355X over 64^2 to 3000 x 2800 cells in 8-, 4- and 2-byte formats,
-    D2Q9 and D2Q9 + D2Q5, with and without links, fitted its constants; the tiles it
-    picks take 2 % longer than the best measured ones on average, 11 % at most):
-      3.5 + 1.5 with links  launch, last store, building the link list
-      rounds x              tiles / 256, rounded up below 2048 tiles, x 3/4 where
-                            two tiles share a CU
-        0.103 per KB of region loaded, 0.15 (+ 0.29 with links) per step,
-        ns / 9 x (0.07, 0.10, 0.17 for 8, 4, 2 bytes) x (waves of cells / 4) per step.
+    steps 2-12 (launches of one run are as even as they come: 7 steps at most 6 at a time are 4 and 3)
+    x rows 4-48 x columns 8-64.  The estimate (us per launch; constants fitted to all those
+    tiles on MI355X over 64^2 to 2500^2 cells in 8-, 4- and 2-byte formats, D2Q9 and
+    D2Q9 + D2Q5, with and without links; the tiles it picks take 2 % longer than the
+    best measured ones on average, 13 % at most; against the fixed tiles before it one of the
+    67 lost, D2Q9 + D2Q5 FP64 on 400^2 cells, 7.1 to 7.4 us):
+      5.3 + 0.8 with links  launch, last store, building the link list
+      rounds x              tiles / 256, rounded up below 2048 tiles; where two tiles share a
+                            CU x 0.78, from 2048 tiles on x 0.68
+        0.13 per KB of region loaded, 0.135 per step,
+        (0.05, 0.07, 0.11 for 8, 4, 2 bytes) x (waves of cells / 4) per step.
     Measured per step, one launch each / fixed tiles of 32 x 32 (FP64 16 x 32) / these:
-    3000 x 2800 FP32 107 / 68 / 63 us, FP64 216 / - / 137 us; 512^2 FP32 6.1 / 2.7 / 2.7 us;
-    128^2 FP64 lid cavity 4.7 / 2.8 / 1.7 us.  Past 2^21 cells (the caches no longer
-    hold them) the estimate is compared with the traffic of single steps at 5.6 TB/s."""
+    3000 x 2800 FP32 107 / 68 / 63 us, FP64 216 / - / 129 us; 512^2 FP32 6.1 / 2.9 / 2.7 us;
+    128^2 FP64 lid cavity 4.7 / 2.8 / 1.7 us; 1000^2 FP64 D2Q9 + D2Q5 - / 35 / 30 us.
+    Past 2^21 cells (the caches no longer hold them) the estimate is compared with the traffic
+    of single steps at 5.6 TB/s, and in runs of 2 steps, which save one launch at most, with 0.87
+    of it and 5 us at least (run(2), single / blocked: 1000^2 FP32 15.5 / 18.2 us per step,
+    2000 x 1500 FP16 19.9 / 23.2; 256^2 8.5 / 6.8)."""
     plane = min((160 * 1024) // (2 * ns * es + 12), 65528 // ((ns - 1) * es) if ns > 1 else 1 << 30)
     half = min((80 * 1024) // (2 * ns * es + 12), plane)
-    per_wave = ns / 9.0 * {8: 0.07, 4: 0.10, 2: 0.17}[es]
+    per_wave = {8: 0.05, 4: 0.07, 2: 0.11}[es]
     best = None
-    for nt in (2, 3, 4, 5, 6, 7, 8, 10, 12):
-        if nt > min(n0, n1):
+    tried = set()
+    for most in (2, 3, 4, 5, 6, 7, 8, 10, 12):
+        if most > min(n0, n1):
             break
+        nt, fewer = most, 0.0   # steps of a launch, share of the launches with one step less
+        launches = nsteps / float(most)
+        if nsteps < LONG_RUN:
+            launches = -(-nsteps // most)
+            nt = -(-nsteps // launches)
+            fewer = nt - nsteps / launches
+        if nt in tried:
+            continue
+        tried.add(nt)
         for tm in {min(t, n0) for t in (4, 8, 12, 16, 20, 24, 32, 40, 48)}:
             for ti in {min(t, n1) for t in (8, 16, 24, 32, 40, 48, 64)}:
-                region = (tm + 2 * nt) * (ti + 2 * nt)
-                if region > plane:
+                if (tm + 2 * nt) * (ti + 2 * nt) > plane:
                     continue
-                tiles = -(-n0 // tm) * -(-n1 // ti)
-                shared = region <= half and tiles > 256
-                rounds = tiles / 256.0
-                if tiles < 2048:
-                    rounds = 2 * math.ceil(tiles / 512.0) if shared else math.ceil(rounds)
-                if shared:
-                    rounds *= 0.75
-                waves = sum(-(-((tm + 2 * s) * (ti + 2 * s)) // 256) for s in range(nt))
-                us = 3.5 + 1.5 * links + rounds * (1.03e-4 * region * ns * es + nt * (0.15 + 0.29 * links)
-                                                   + per_wave * waves)
-                key = (us / nt, nt, tm, ti)
+                us = 0.0
+                for q, share in ((nt, 1.0 - fewer), (nt - 1, fewer)):
+                    if share == 0.0:
+                        continue
+                    region = (tm + 2 * q) * (ti + 2 * q)
+                    tiles = -(-n0 // tm) * -(-n1 // ti)
+                    shared = region <= half and tiles > 256
+                    rounds = tiles / 256.0
+                    if tiles < 2048:
+                        rounds = 2 * math.ceil(tiles / 512.0) if shared else math.ceil(rounds)
+                    if shared:
+                        rounds *= 0.78 if tiles < 2048 else 0.68
+                    waves = sum(-(-((tm + 2 * s) * (ti + 2 * s)) // 256) for s in range(q))
+                    us += share * (5.3 + 0.8 * links + rounds * (1.3e-4 * region * ns * es + q * 0.135
+                                                                  + per_wave * waves))
+                key = (us * launches / nsteps, nt, tm, ti)
                 if best is None or key < best:
                     best = key
-    if best is None or (n0 * n1 > 1 << 21 and best[0] >= n0 * n1 * 2.0 * ns * es / 5.6e6):
+    single = 2.0 * n0 * n1 * ns * es / 5.6e6
+    if nsteps <= 2:
+        single = max(5.0, 0.87 * single)
+    elif n0 * n1 <= 1 << 21:
+        single = math.inf
+    if best is None or best[0] >= single:
         return None
     return best[1:]
 
@@ -802,7 +828,7 @@ class Simulation:
         c = self.container
         self.params.t = self.t
         parity = ctypes.c_int(0)
-        tb = self._blocking_shape() if fold and nsteps > 1 else None
+        tb = self._blocking_shape(nsteps) if fold and nsteps > 1 else None
         if tb is not None:
             nt, tm, ti = tb
             self._check(self.module.lbm_gen_run_blocked(ctypes.c_void_p(c.F.ptr), ctypes.c_void_p(c.Fnew.ptr),
@@ -827,9 +853,9 @@ class Simulation:
         self.nt += nsteps
         self.t = self.t + nsteps * self.dt
 
-    def _blocking_shape(self):
-        """(steps per launch, tile rows, tile columns) of the temporally blocked run, or
-        None: 1D and 2D schemes on the wrap path (periodic, or every list folded with
+    def _blocking_shape(self, nsteps=LONG_RUN):
+        """(steps per launch, tile rows, tile columns) of the temporally blocked run of
+        nsteps steps, or None: 1D and 2D schemes on the wrap path (periodic, or every list folded with
         its table sources within one cell) with velocity components in {-1, 0, 1}.
         The tile and its halo live in LDS (_blocked_tile)."""
         if not self.temporal_blocking or self.dim > 2 or not self._wrap or not self._unit_velocities:
@@ -845,7 +871,7 @@ class Simulation:
                 return None
             nt = min(nt, nin[0])
             return (nt, 1, min(ti, nin[0])) if nt >= 2 else None
-        return _blocked_tile(self.ns, es, nin[0], nin[1], bool(self.params.bbmask))
+        return _blocked_tile(self.ns, es, nin[0], nin[1], bool(self.params.bbmask), min(int(nsteps), LONG_RUN))
 
     def sync(self):
         self.rt.sync()
