@@ -1268,8 +1268,8 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   const C* cref = a.cref;
   (void)cref;
   // TB_BATCH cells per thread in flight: all their loads are issued before the first
-  // is written to LDS (2-byte and 4-byte formats without links 1 to 3 % faster than one at a
-  // time; FP64 2 % slower: 1000^2 D2Q9 + D2Q5 35.7 us per step with 2, 35.1 with 1)
+  // is written to LDS (2-byte and 4-byte formats without links 1 to 3 %% faster than one at a
+  // time; FP64 2 %% slower: 1000^2 D2Q9 + D2Q5 35.7 us per step with 2, 35.1 with 1)
   for (int c0 = threadIdx.x; c0 < RN; c0 += TB_BATCH * blockDim.x) {
     S v[TB_BATCH][NS];
     uint32_t bits_[TB_BATCH];
