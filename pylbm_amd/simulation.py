@@ -70,17 +70,17 @@ def _blocked_tile(ns, es, n0, n1, links, nsteps):
     steps per launch share the launch and the load but recompute the halo, small tiles
     fill the GPU but have more halo, two workgroups share a CU when a region fits half
     its LDS.  The tile is the one whose estimated time per step is the least of
-    steps 2-12 (launches of one run are as even as they come: 7 steps at most 6 at a time are 4 and 3)
-    x rows 4-48 x columns 8-64.  The estimate (us per launch; constants fitted to all those
-    tiles on MI355X over 64^2 to 2500^2 cells in 8-, 4- and 2-byte formats, D2Q9 and
-    D2Q9 + D2Q5, with and without links; the tiles it picks take 2 % longer than the
-    best measured ones on average, 13 % at most; against the fixed tiles before it one of the
-    67 lost, D2Q9 + D2Q5 FP64 on 400^2 cells, 7.1 to 7.4 us):
-      5.3 + 0.8 with links  launch, last store, building the link list
+    steps 2-12 (launches of one run are as even as they come: 7 steps at most 6 at a time are
+    4 and 3) x rows 4-48 x columns 8-64.  The estimate (us per launch; constants fitted to all
+    those tiles on MI355X over 64^2 to 3000 x 2800 cells in 8-, 4- and 2-byte formats, D2Q9 and
+    D2Q9 + D2Q5, with and without links; the tiles it picks take 1.5 % longer than the
+    best measured ones on average, 11 % at most; against the fixed tiles before it one grid
+    of 76 lost, D2Q9 + D2Q5 FP64 on 400^2 cells, 7.1 to 7.4 us):
+      3.2 + 1.5 with links  launch, last store, building the link list
       rounds x              tiles / 256, rounded up below 2048 tiles; where two tiles share a
-                            CU x 0.78, from 2048 tiles on x 0.68
-        0.13 per KB of region loaded, 0.135 per step,
-        (0.05, 0.07, 0.11 for 8, 4, 2 bytes) x (waves of cells / 4) per step.
+                            CU x 0.75, from 2048 tiles on x 0.63
+        0.115 per KB of region loaded, 48 B more per row for its partial lines, 0.18 per step,
+        (0.02, 0.015, 0.09 for 8, 4, 2 bytes) x (waves of cells / 4) per step.
     Measured per step, one launch each / fixed tiles of 32 x 32 (FP64 16 x 32) / these:
     3000 x 2800 FP32 107 / 68 / 63 us, FP64 216 / - / 129 us; 512^2 FP32 6.1 / 2.9 / 2.7 us;
     128^2 FP64 lid cavity 4.7 / 2.8 / 1.7 us; 1000^2 FP64 D2Q9 + D2Q5 - / 35 / 30 us.
@@ -90,7 +90,7 @@ def _blocked_tile(ns, es, n0, n1, links, nsteps):
     2000 x 1500 FP16 19.9 / 23.2; 256^2 8.5 / 6.8)."""
     plane = min((160 * 1024) // (2 * ns * es + 12), 65528 // ((ns - 1) * es) if ns > 1 else 1 << 30)
     half = min((80 * 1024) // (2 * ns * es + 12), plane)
-    per_wave = {8: 0.05, 4: 0.07, 2: 0.11}[es]
+    per_wave = {8: 0.02, 4: 0.015, 2: 0.09}[es]
     best = None
     tried = set()
     for most in (2, 3, 4, 5, 6, 7, 8, 10, 12):
@@ -120,10 +120,10 @@ def _blocked_tile(ns, es, n0, n1, links, nsteps):
                     if tiles < 2048:
                         rounds = 2 * math.ceil(tiles / 512.0) if shared else math.ceil(rounds)
                     if shared:
-                        rounds *= 0.78 if tiles < 2048 else 0.68
+                        rounds *= 0.75 if tiles < 2048 else 0.63
                     waves = sum(-(-((tm + 2 * s) * (ti + 2 * s)) // 256) for s in range(q))
-                    us += share * (5.3 + 0.8 * links + rounds * (1.3e-4 * region * ns * es + q * 0.135
-                                                                  + per_wave * waves))
+                    loaded = (tm + 2 * q) * ((ti + 2 * q) * es + 48) * ns
+                    us += share * (3.2 + 1.5 * links + rounds * (1.15e-4 * loaded + q * 0.18 + per_wave * waves))
                 key = (us * launches / nsteps, nt, tm, ti)
                 if best is None or key < best:
                     best = key
