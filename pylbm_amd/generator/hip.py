@@ -1188,7 +1188,7 @@ _TB_KERNEL = r"""// ------------------------------------------------ temporally 
 // after the other, made the launch as slow as the tile with most of them (per step,
 // entries in the cells / in the list: 901 x 219 channel around a cylinder,
 // interpolated walls, FP32 deviations 5.8 / 3.4 us; with plain walls, 1024 x 256 FP32
-// 3.8 / 3.5 us; 5000-cell 1D shock tube FP64 1.4 / 0.77 us).
+// 3.8 / 3.4 us; 5000-cell 1D shock tube FP64 1.4 / 0.65 us).
 // A region with more links than the list holds takes the mask, table bits and first
 // entries of its cells into LDS and substitutes link by link in the cell.
 template <typename C>
@@ -1367,9 +1367,9 @@ _PAIR_KERNEL = r"""// ------------------------------------------------ two steps
 // 32 cells are 128 B of FP32; 13 rows and their halo are 510 of 512 threads, two
 // workgroups to a CU in 128 registers.  FP64 needs more registers (two workgroups: 75
 // spilled, 605 us per step of 150 x 201 x 183) and has a CU for one workgroup of 16 rows in
-// 168, with folded links 13 rows in 256.  What bounds it now: 256^3 FP32 at 306 us per step
+// 168, with folded links 13 rows in 256.  What bounds it now: 256^3 FP32 at 308 us per step
 // moves 4.4 TB/s of HBM traffic (1.1 reads and 1 write per population and two steps) with
-// the vector units 43 %% busy; the rest are the barriers of two workgroups per CU.
+// the vector units under half busy; the rest are the barriers of two workgroups per CU.
 template <typename C>
 struct PairArgs {
   int32_t tiles_i, tiles_m, ty, nz;   // tiles along the inner and mid axes, rows of a tile, planes per workgroup
@@ -1583,9 +1583,10 @@ static int pair_launch(const void* f, void* fn, const lbm_layout* L, lbm_params*
 // along the outer axis: nz + 2 planes per workgroup at so many us per plane with few
 // workgroups, one or two on every CU, a little more in long chunks, whose neighbours
 // drift apart in the L2 (constants fitted to a sweep of 19 grids, 80^3 to 256^3, with and
-// without folded links, FP32 and FP64 D3Q19 on MI355X: 5 % rms).  Per step, one at a time /
-// two: 256^3 FP32 452 / 306 us, 128^3 59 / 47, 80^3 18 / 19; 150 x 201 x 183 FP64 310 / 205,
-// 80^3 31 / 24; 256 x 128 x 128 with spheres FP32 117 / 99, FP64 222 / 170.
+// without folded links, FP32 and FP64 D3Q19 on MI355X: 5 %% rms).  Per step, one at a time /
+// two: 256^3 FP32 448 / 308 us, 128^3 53 / 48, 80^3 16 / 19; 150 x 201 x 183 FP64 310 / 206,
+// 96^3 45 / 35; 256 x 128 x 128 with spheres FP32 118 / 100, FP64 222 / 174; 200^3 D3Q15 FP32
+// 192 / 142, FP64 335 / 238, D3Q6 FP32 70 / 56, FP64 131 / 89.
 template <typename S, bool MASK>
 static int pair_planes(const int32_t (&nin)[3]) {
   constexpr double part = NS / 19.0;
@@ -1612,16 +1613,16 @@ static int pair_planes(const int32_t (&nin)[3]) {
   return planes;
 }
 
-// whether the compiler spilled registers of the kernel to scratch memory: a reload there waits
-// for every load in flight, and single steps are faster (D3Q19 FP64 with a source term of sines
-// of X, Y, Z and t, 10 registers spilled: 200^3 421 us per step one at a time, 468 in pairs; a
-// source linear in X, Y and Z fits: 424 and 354; 96^3 with few workgroups 51 and 51)
+// whether the compiler spilled more than a few registers of the kernel to scratch memory: a
+// reload there waits for every load in flight (200^3 D3Q19 FP64, us per step one at a time /
+// in pairs: source terms in t, 12 B spilled, 420 / 315; linear in X, Y and Z, 8 B, 421 / 354; sines
+// of X, Y, Z and t, 44 B, 421 / 468)
 template <typename S, bool MASK>
 static bool pair_spills() {
   static const bool spills = [] {
     hipFuncAttributes at;
     const hipError_t e = hipFuncGetAttributes(&at, (const void*)pair_step<S, MASK, pair_rows<S, MASK>()>);
-    return e != hipSuccess || at.localSizeBytes > 0;
+    return e != hipSuccess || at.localSizeBytes > 24;
   }();
   return spills;
 }

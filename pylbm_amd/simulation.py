@@ -47,13 +47,15 @@ LBM_F64 = rtm.LBM_F64
 # save their launches.  With Neumann lists, which fold in no other way, the table takes
 # the place of the ghost fill and every launch, and is four times as large: 240 x 112 x 112
 # duct, 125,440 entries on its inflow and outflow faces, FP32 118 us per step in launches,
-# 93 us folded; FP64 198 and 159.
+# 93 us folded; FP64 198 and 159.  So it is with spheres in the box and one outflow face:
+# 160 x 128 x 128 FP32 102 and 78, 256 x 160 x 160 252 and 185; FP64 184 and 147, 441 and 371;
+# FP16 64 and 47, 165 and 141.
 FOLD_TABLE_MAX = 1 << 16
 # Temporally blocked run in 1D: (steps per launch, cells per tile); a tile and its halo
 # of steps cells on both sides fill one region of TB_PLANE_1D cells (the generated
 # module's constant of the same name).  A 1D step is launch and latency: the 5000-cell
 # FP64 shock tube (3 x D1Q2, Neumann ends) takes 4.1 us per step with one launch each
-# and 0.77 us this way.
+# and 0.65 us this way.
 TB_SHAPE_1D = (64, 128)
 TB_PLANE_1D = 256
 # Steps of a run from which on the evenness of its launches no longer matters to their number
