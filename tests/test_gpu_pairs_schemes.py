@@ -36,26 +36,28 @@ def _box(shape, scheme, walls):
     return d
 
 
-def _start(d, dtype):
-    sim = Simulation(d, dtype=dtype)
-    rng = np.random.default_rng(12)
-    for k in range(sim.ns):
-        sim.F_halo[k] = sim.F_halo[k] * (1.0 + 0.05 * rng.standard_normal(sim.domain.shape_halo))
-    return sim
+def _state(sim):
+    return sim.container.F.fields_raw()[(slice(None),) + (slice(1, -1),) * 3]
 
 
 def _same_bits(d, dtype, steps, launches):
-    ref, sim = _start(d, dtype), _start(d, dtype)
+    ref, sim = Simulation(d, dtype=dtype), Simulation(d, dtype=dtype)
+    rng = np.random.default_rng(12)
+    for c in ref.scheme.consm:   # rough conserved moments, and with the sources' first step off equilibrium
+        ref.m_halo[c] = ref.m_halo[c] + 0.02 * rng.standard_normal(ref.domain.shape_halo)
+    ref.equilibrium()
+    ref.m2f()
+    ref.sync()
+    sim.container.F.copy_from(ref.container.F)
     for _ in range(steps):
         ref.one_time_step()
     first = sim.container.F.ptr
     sim.run(steps)
     assert (sim.container.F.ptr != first) == (launches % 2 == 1)
     assert sim.t == ref.t
-    for k in range(sim.ns):
-        want = ref.F[k]
-        assert np.isfinite(want).all()
-        assert np.array_equal(sim.F[k], want), k
+    want = _state(ref)
+    assert np.isfinite(want).all()
+    assert np.array_equal(_state(sim), want)
 
 
 @pytest.mark.parametrize("shape,dtype,walls", [((97, 130, 159), "float32", False), ((77, 190, 93), "float64", False),
