@@ -566,17 +566,20 @@ __host__ __device__ constexpr int block_rows() {
 }
 
 // Waves per SIMD of a fused step.  FP64 in 3D, at least 4: source terms in X, Y, Z and t
-// bring D3Q19 to 129 registers, one more than 4 waves have (200^3 431 us per step with 3).
-// 2-byte formats in 3D with stores past the caches, at most 5: with 6, 200^3 FP16 takes 135
-// us instead of 129, 230 x 210 x 220 164 instead of 158; 16 populations and more (6
-// populations stream faster with all 8, 200^3 47 us instead of 58).
+// bring D3Q19 to 129 registers, one more than 4 waves have (200^3 432 us per step with 3, 421).
+// Stores past the caches in 3D, 16 populations and more, where more waves stream slower: 2-byte
+// formats and FP32 at most 5 (with 6, 200^3 FP16 takes 135 us instead of 129, 230 x 210 x 220 164
+// instead of 158, 144^3 FP32 86.0 instead of 84.7; 6 populations stream faster with all 8, 200^3
+// FP16 47 us instead of 58); FP32 with four cells per thread at most 2 (with 3, 200^3 240 us
+// instead of 237, 230 x 210 x 220 313 instead of 307).
 template <typename S, bool TABLE>
 constexpr int least_waves() {
   return sizeof(S) == 8 && DIM == 3 && NS <= 19 && !TABLE ? 4 : 1;
 }
-template <typename S, bool NT>
+template <typename S, int VEC, bool NT>
 constexpr int most_waves() {
-  return sizeof(S) == 2 && DIM == 3 && NS >= 16 && NT ? 5 : 8;
+  if (DIM < 3 || NS < 16 || !NT) return 8;
+  return sizeof(S) == 2 ? 5 : Codec<S>::kind == LBM_F32 ? (VEC > 1 ? 2 : 5) : 8;
 }
 
 template <typename S>
@@ -636,7 +639,7 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t 
 // batched loads take registers (D2Q9 FP64 48 -> 130) that boxes without a table need not pay.
 template <typename S, bool FOLD, int VEC, typename I, bool NT, bool TABLE>
 __global__ void __launch_bounds__(LBM_BX * block_rows<S>())
-__attribute__((amdgpu_waves_per_eu(least_waves<S, TABLE>(), most_waves<S, NT>())))
+__attribute__((amdgpu_waves_per_eu(least_waves<S, TABLE>(), most_waves<S, VEC, NT>())))
 fused_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Codec<S>::C> a) {
   using C = typename Codec<S>::C;
   // full-value arithmetic for FP64 (as pylbm), deviations from the rest state otherwise
@@ -1919,22 +1922,26 @@ def generate_source(spec: KernelSpec) -> str:
     vstores = ["vstore<S, VEC, NT>(fn + ((I)a.dst_off[%d] + cell), G%d);" % (k, k) for k in range(ns)]
 
     # The arithmetic of the step.  Contracted, moments share partial sums and a product and a
-    # sum of one statement become one FMA: up to a quarter fewer instructions.  FP64 does
-    # (errors against wider arithmetic, replayed on the CPU over 32 flows of 30 to 400 steps,
-    # relative to single roundings: momentum 0.83 in D3Q19, 0.96 in D2Q9; 128^3 in pairs 84 ->
-    # 78 us per step), and so do the 2-byte formats in 3D, whose stored values round 2^13
-    # times more coarsely (momentum 1.00 over 128 flows; 128^3 27.0 -> 25.2 us), but for M^-1 m:
-    # a product there enters several populations, and fused it rounds differently in each of their sums.
-    # FP32 and its deviations round every product and sum on its own: deviations get their
-    # accuracy from their arithmetic (contracted 1.07, shared sums alone 1.03; 256^3 Taylor-
-    # Green vortex after 1000 steps 4.7e-7 against 3.9e-7, 306 us per step either way), and FP32
-    # gains 1 to 3 % in pairs (256^3 308 -> 305 us) and loses as much in single steps of large
-    # boxes (230 x 210 x 220 308 -> 317 us).
-    fuse, fuse_16 = not rel, not rel and dim == 3
+    # sum of one statement become one FMA: up to a quarter fewer instructions.  Errors
+    # against wider arithmetic, replayed on the CPU over 32 to 128 flows of 30 to 400 steps,
+    # relative to single roundings (density, momentum):
+    #   FP64 0.74, 0.83 (D3Q19), 0.97, 0.96 (D2Q9): contracted; 128^3 in pairs 84 -> 78 us;
+    #   FP32 in 3D 0.99, 0.99: contracted, and the increment is added to the stored value
+    #   itself; 256^3 in pairs 308 -> 305 us per step, 80^3 15.7 -> 15.2;
+    #   2-byte formats in 3D 1.01, 1.00: contracted but for M^-1 m, where a product enters several
+    #   populations and, fused, rounds differently in each of their sums; 128^3 27.0 -> 25.2 us;
+    #   FP32 deviations in 3D 1.05, 1.07 (shared sums alone 1.07, 1.03; 256^3 Taylor-Green vortex
+    #   after 1000 steps 4.7e-7 against 3.9e-7): not contracted, their accuracy is that of
+    #   their arithmetic, and it costs them nothing (306 us per step of 256^3 either way).
+    # The FP32-compute formats of 1D and 2D schemes are not contracted either and keep the
+    # results they have always had bit for bit (contracted: momentum 0.97 FP32, 0.99
+    # deviations; 1024 x 256 channel 634 us per 200 steps instead of 670).
+    fuse, fuse_dev = not rel, not rel and dim == 3
 
-    def step_lines(on, dev):
-        """f2m, collision and m2f of one cell, contracted (on) or not, in deviations (dev)
-        or full values."""
+    def step_lines(dev, on, on_back, added=False):
+        """f2m, collision and m2f of one cell in deviations (dev) or full values, f2m and
+        collision contracted (on), m2f contracted (on_back); added: the increments are
+        added to the stored values."""
         b1 = _SumBuilder("p", on)
         f2m = _transform(b1, M, fvars, mvars, ksym, sig_f2m)
         out = (["#pragma clang fp contract(on)"] if on else []) + b1.lines + ["C %s = %s;" % (o, e) for o, e in f2m]
@@ -1948,16 +1955,21 @@ def generate_source(spec: KernelSpec) -> str:
         b2 = _SumBuilder("rd" if dev else "r", on)
         m2f = _inverse_transform(b2, iM, names, ["g%d" % k for k in range(ns)], ksym, sig_m2f, tag="d" if dev else "")
         back = b2.lines + ["const C %s = %s;" % (o, e) for o, e in m2f]
-        if dev:
-            back += ["G%d[j] = Codec<S>::encode_dev(f%d + g%d, a.wshift[%d]);" % (k, k, k, k) for k in range(ns)]
-        else:
-            back += ["G%d[j] = Codec<S>::encode(g%d, a.wshift[%d]);" % (k, k, k) for k in range(ns)]
-        return out + coll + (["{", "#pragma clang fp contract(off)"] + back + ["}"] if on and dev else back)
-    collide = ["if constexpr (%s) {" % ("DEV && sizeof(S) > 2" if fuse_16 else "DEV")]
-    collide += ["  " + ln for ln in step_lines(False, True)]
-    if fuse_16:
-        collide += ["} else if constexpr (DEV) {"] + ["  " + ln for ln in step_lines(True, True)]
-    collide += ["} else {"] + ["  " + ln for ln in step_lines(fuse, False)] + ["}"]
+        form = "L{0}[j] + g{0}" if added else \
+            "Codec<S>::encode_dev(f{0} + g{0}, a.wshift[{0}])" if dev else "Codec<S>::encode(g{0}, a.wshift[{0}])"
+        back += [("G{0}[j] = " + form + ";").format(k) for k in range(ns)]
+        return out + coll + (["{", "#pragma clang fp contract(off)"] + back + ["}"] if on and not on_back else back)
+
+    cases = [("DEV", step_lines(True, False, False)), (None, step_lines(False, fuse, fuse))]
+    if fuse_dev:
+        cases = [("Codec<S>::kind == LBM_F32D", step_lines(True, False, False)),
+                 ("Codec<S>::kind == LBM_F32", step_lines(True, True, True, added=True)),
+                 ("DEV", step_lines(True, True, False)), cases[1]]
+    collide = []
+    for test, lines in cases:
+        collide.append(("} else " if collide else "") + ("if constexpr (%s) {" % test if test else "{"))
+        collide += ["  " + ln for ln in lines]
+    collide.append("}")
 
     # ---------------------------------------------------------- f2m / m2f / eq
     b3 = _SumBuilder("p")
