@@ -281,9 +281,10 @@ typedef struct lbm_params {
    * round-robin order, -1 = the default (1 on the halo path, 0 on the wrap path) */
   int32_t xcd_remap;
   /* cells per thread of the step along the contiguous axis: 0 = the default (4
-   * for the 2- and 4-byte formats where that leaves >= 2^20 threads, else 1),
-   * 1 = one cell per thread, 4 = four (the contiguous interior extent must be a
-   * multiple of 4); every choice gives the same bits */
+   * for the 4-byte formats on the wrap path without folded links, where that leaves
+   * >= 2^20 threads and the stores bypass the caches, else 1), 1 = one cell per
+   * thread, 4 = four (2- and 4-byte formats; the contiguous interior extent must be a
+   * multiple of 4; with table entries one all the same); every choice gives the same bits */
   int32_t vec_cells;
   /* lbm_gen_run on the wrap path: 0 = two steps per launch where that is the faster
    * (3D), 1 = one step per launch; the same bits */

@@ -84,8 +84,8 @@ def _blocked_tile(ns, es, n0, n1, links, nsteps):
         0.115 per KB of region loaded, 48 B more per row for its partial lines, 0.18 per step,
         (0.02, 0.015, 0.09 for 8, 4, 2 bytes) x (waves of cells / 4) per step.
     Measured per step, one launch each / fixed tiles of 32 x 32 (FP64 16 x 32) / these:
-    3000 x 2800 FP32 107 / 68 / 63 us, FP64 216 / - / 129 us; 512^2 FP32 6.1 / 2.9 / 2.7 us;
-    128^2 FP64 lid cavity 4.7 / 2.8 / 1.7 us; 1000^2 FP64 D2Q9 + D2Q5 - / 35 / 30 us.
+    3000 x 2800 FP32 107 / 68 / 61 us, FP64 216 / - / 129 us; 512^2 FP32 6.1 / 2.9 / 2.7 us;
+    128^2 FP64 lid cavity 4.7 / 2.8 / 1.7 us; 1000^2 FP64 D2Q9 + D2Q5 - / 35 / 31 us.
     Past 2^21 cells (the caches no longer hold them) the estimate is compared with the traffic
     of single steps at 5.6 TB/s, and in runs of 2 steps, which save one launch at most, with 0.87
     of it and 5 us at least (run(2), single / blocked: 1000^2 FP32 15.5 / 18.2 us per step,
