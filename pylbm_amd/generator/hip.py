@@ -1625,6 +1625,7 @@ static bool pair_spills() {
   static const bool spills = [] {
     hipFuncAttributes at;
     const hipError_t e = hipFuncGetAttributes(&at, (const void*)pair_step<S, MASK, pair_rows<S, MASK>()>);
+    if (e != hipSuccess) (void)hipGetLastError();   // single steps; not the next launch's error
     return e != hipSuccess || at.localSizeBytes > 24;
   }();
   return spills;
