@@ -499,7 +499,7 @@ using namespace lbm;
 #define TB_MAX_NT (DIM == 1 ? 64 : 16) // steps per temporally blocked launch, at most
 #define TB_PLANE_1D 256                // cells of a 1D region, at most
 #define TB_MASK %(bbsub_ok)d                    // folded links possible
-#define TB_BATCH (sizeof(S) == 8 ? 1 : 2)   // cells a thread of a blocked workgroup loads at once
+#define TB_BATCH (sizeof(S) == 8 && DIM == 2 ? 1 : 2)   // cells a thread of a blocked workgroup loads at once
 #define TB_LINKS 4                     // folded links a thread of a blocked workgroup holds
 #define PAIR_OK %(pair_ok)d            // the two-step kernel is generated
 
@@ -1272,7 +1272,7 @@ tb_step(const S* __restrict__ f, S* __restrict__ fn, const StepArgs<typename Cod
   (void)cref;
   // TB_BATCH cells per thread in flight: all their loads are issued before the first
   // is written to LDS (2-byte and 4-byte formats without links 1 to 3 %% faster than one at a
-  // time; FP64 2 %% slower: 1000^2 D2Q9 + D2Q5 35.7 us per step with 2, 35.1 with 1)
+  // time; FP64 in 2D 2 %% slower: 1000^2 D2Q9 + D2Q5 35.7 us per step with 2, 35.1 with 1)
   for (int c0 = threadIdx.x; c0 < RN; c0 += TB_BATCH * blockDim.x) {
     S v[TB_BATCH][NS];
     uint32_t bits_[TB_BATCH];
